@@ -740,6 +740,11 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
     // reverse time at 512x512x256, chunks of 32; 2 % more at 96x96x64, chunks of 8)
     const bool march_mu = march && (xc_a >= 16 || (sv && std::strcmp(sv, "march") == 0));
     const int64_t step0 = c->step;
+    // the FP32 adjoint keeps the population kernels' forward trajectory: d J / d kappa sums
+    // terms that nearly cancel, and a trajectory rounded in another order moves it by more
+    // (up to 3e-4) than the form's stated accuracy
+    const bool moments = c->moments;
+    if (c->form == CPMP_FORM_FP32) c->moments = false;
     const size_t fbytes = 19 * (size_t)N * c->pop_bytes, rbytes = (size_t)N * c->scal_bytes;
     const size_t hb = c->form == CPMP_FORM_FP64 ? sizeof(double) : sizeof(float);   // population cotangents
     // tape entry of step n, in the storage scalar type (FP64 or FP32): rho^n after
@@ -793,18 +798,15 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
             hipError_t e = hipMemcpyAsync(c->f[c->cur], src, fbytes, hipMemcpyDeviceToDevice, c->stream);
             return e != hipSuccess ? e : hipMemcpyAsync(c->rho, src + fbytes, rbytes, hipMemcpyDeviceToDevice, c->stream);
         };
-        // one forward step that records its tape entry tr
-        auto taped_step = [&](char *tr) -> hipError_t {
-            hipError_t e;
-            if ((e = launch_wall(c)) != hipSuccess) return e;
-            if ((e = launch_mu(c, tr)) != hipSuccess) return e;   // also copies rho (after the wall fill) to tr
-            if ((e = launch_collide(c, false, tr + N * sb)) != hipSuccess) return e;
-            return launch_macro(c);
-        };
+        // a run of L forward steps that record their tape entries
         auto tape_steps = [&](char *tp, int L) -> hipError_t {
             for (int k = 0; k < L; ++k) {
-                const hipError_t e = taped_step(tp + k * q.per_tape);
-                if (e != hipSuccess) return e;
+                char *tr = tp + k * q.per_tape;
+                hipError_t e;
+                if ((e = launch_wall(c)) != hipSuccess) return e;
+                if ((e = launch_mu(c, tr)) != hipSuccess) return e;   // also copies rho (after the wall fill) to tr
+                if ((e = launch_collide(c, false, tr + N * sb, false, k == 0, k == L - 1)) != hipSuccess) return e;
+                if ((e = launch_macro(c)) != hipSuccess) return e;
             }
             return hipSuccess;
         };
@@ -862,7 +864,7 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
         for (int sg = 0; sg < q.nseg; ++sg) {
             AHIP(save(ckpt + sg * q.per_ck));
             const int L = std::min(q.C, q.n0 - sg * q.C);
-            for (int k = 0; k < L; ++k) AHIP(launch_step(c, false));
+            AHIP(launch_steps(c, L, false));
         }
         AHIP(tape_steps(tape, q.ntaped));
         AHIP(save(fin));
@@ -918,7 +920,7 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
                 }
                 // first pass: sub-checkpoints at S, 2S, .. (nsub-2)S, last sub-segment taped
                 for (int j = 1; j < nsub; ++j) {
-                    for (int k = 0; k < S; ++k) AHIP(launch_step(c, false));
+                    AHIP(launch_steps(c, S, false));
                     if (j <= nsub - 2) AHIP(save(subck + (j - 1) * q.per_ck));
                 }
                 const int Llast = L - (nsub - 1) * S;
@@ -950,6 +952,7 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
     c->mv_valid = false;
 done:
     c->stream = s;
+    c->moments = moments;
     if (s2) {
         (void)hipStreamSynchronize(s2);
         (void)hipStreamDestroy(s2);

@@ -288,15 +288,25 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
     if (hipMalloc(&c->mu, c->N * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "mu");
     const char *fuse = std::getenv("CPMP_FUSE");
     size_t ring_elems = 0, chunk_elems = 0;
-    // every storage form sums the density inside the march collide where the tiles
-    // cover the lattice (not with the one-thread-per-node collide of small FP64 lattices)
-    if (!c->collide_v1 && !(fuse && std::strcmp(fuse, "0") == 0) &&
-        fuse_geometry(p->nx, p->ny, p->nz, c->dp.xc, &ring_elems, &chunk_elems)) {
+    const bool fuse_off = fuse && std::strcmp(fuse, "0") == 0;
+    const bool covered = fuse_geometry(p->nx, p->ny, p->nz, c->dp.xc, &ring_elems, &chunk_elems);
+    c->moments = moment_path(*p, c->dp, fuse_off, covered);
+    if (c->moments) {
+        c->collide_v1 = false;
+        c->step_chunk = moment_chunk(p->nx, p->ny, p->nz, p->form);
         if (hipMalloc(&c->rho_next, c->N * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "next rho");
+        c->fuse_bytes = (size_t)c->N * c->scal_bytes;
+    }
+    // the population march sums the density inside the collide where the tiles cover the
+    // lattice (not the one-thread-per-node collide of small FP64 lattices).  The adjoint of
+    // the FP32 form runs it also where runs of steps take the moments.
+    if (!c->collide_v1 && !fuse_off && covered && (!c->moments || c->form == CPMP_FORM_FP32)) {
+        if (!c->rho_next && hipMalloc(&c->rho_next, c->N * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "next rho");
         if (hipMalloc(&c->rbuf, ring_elems * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "tile rings");
         if (hipMalloc(&c->cbuf, chunk_elems * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "chunk planes");
         c->fuse_bytes = ((size_t)c->N + ring_elems + chunk_elems) * c->scal_bytes;
-        // the fused path stores populations tile-contiguous (pop_site)
+    }
+    if (covered && !fuse_off && !c->collide_v1) {   // populations tile-contiguous (pop_site)
         c->dp.tiled = 1;
         c->dp.nty = p->ny / kTileY;
         c->dp.ntz = p->nz / kTileZ;
@@ -439,6 +449,7 @@ int cpmp_step(cpmp_ctx *c, int nsteps) {
     if (nsteps == 0) return CPMP_OK;
     HIPCHK(hipSetDevice(c->p.device));
     HIPCHK(launch_steps(c, nsteps));
+    c->step += nsteps;
     HIPCHK(hipStreamSynchronize(c->stream));
     c->mv_valid = true;
     return CPMP_OK;
@@ -644,6 +655,7 @@ int cpmp_time_steps(cpmp_ctx *c, int nsteps, double *ms) {
     HIPCHK(hipStreamSynchronize(c->stream));
     HIPCHK(hipEventRecord(a, c->stream));
     HIPCHK(launch_steps(c, nsteps));
+    c->step += nsteps;
     HIPCHK(hipEventRecord(b, c->stream));
     HIPCHK(hipEventSynchronize(b));
     float t = 0;
@@ -675,7 +687,7 @@ int cpmp_kernel_times(cpmp_ctx *c, int nsteps, double *ms, int *launches) {
         HIPCHK(launch_mu(c));
         HIPCHK(hipEventRecord(ev[3], c->stream));
         HIPCHK(hipEventRecord(ev[4], c->stream));
-        HIPCHK(launch_collide(c, n == nsteps - 1));
+        HIPCHK(launch_collide(c, n == nsteps - 1, nullptr, false, n == 0, n == nsteps - 1));
         HIPCHK(hipEventRecord(ev[5], c->stream));
         HIPCHK(hipEventRecord(ev[6], c->stream));
         HIPCHK(launch_macro(c));

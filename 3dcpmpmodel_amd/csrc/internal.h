@@ -71,6 +71,8 @@ struct cpmp_ctx {
     unsigned band_cap = 0;      // descriptor slots
     int band_par = 0;
     bool collide_v1 = false;    // one-thread-per-node collide (node_collide)
+    bool moments = false;       // runs of steps carry 13 moments per node (moment_path)
+    int step_chunk = 0;         // x planes per workgroup of the moment step
     size_t fuse_bytes = 0;
     double *mv = nullptr;       // 3*N, MV of the last step
     double *mu_w = nullptr;     // 2*NXY: bottom then top
@@ -100,6 +102,21 @@ int march_chunk(int nx, int ny, int nz, int form);
 // the one-thread-per-node collide instead of the x march (CPMP_COLLIDE=v1 / march
 // override): FP64 lattices too small for 2048 march workgroups of 2 planes
 bool node_collide(int nx, int ny, int nz, int form);
+// runs of steps hand 12 moments per node and the density from one step to the next
+// (the reference's unit rates; not the FP16 form, whose state is defined by its stored
+// populations).  Lattices below 100 000 nodes keep the population kernels: there a step
+// is a few launches' latency, and the march takes longer from end to end than a launch of
+// one thread per node (us per step, population kernels against moments: 64x1x32 FP64
+// 19.0 / 20.1, 32^3 FP64 17.6 / 22.1, 48x40x36 FP32 27.9 / 30.9; 64^3 FP64 40.2 / 35.9,
+// FP32 34.5 / 30.5, 96x96x64 FP32 65.9 / 47.6).  CPMP_COLLIDE=march or CPMP_XC take the
+// moments on any lattice; CPMP_COLLIDE=v1 and, on lattices the march tiles cover,
+// CPMP_FUSE=0 keep the populations.
+bool moment_path(const cpmp_params &p, const DevParams &d, bool fuse_off, bool covered);
+constexpr int kMomentFields = 12;
+int moment_chunk(int nx, int ny, int nz, int form);
+// one collide and stream step from the current set into the other: populations or
+// moments in and out; rho_next receives the new density of the fluid nodes
+hipError_t launch_moment_step(cpmp_ctx *c, bool in_pops, bool out_pops, bool want_mv, void *uout);
 constexpr int kTileY = 8, kTileZ = 32;   // in-plane tile of the march kernels and of tiled population storage
 constexpr int kWallTile = 16;             // columns per edge of the wall-fill tiles (16 x 16 workgroups)
 // copy one population set between the device layout and the reference node order
@@ -107,11 +124,12 @@ hipError_t launch_pop_relayout(cpmp_ctx *c, const void *src, void *dst, bool to_
 // uout (when given): u, grad mu, grad rho of every node, 9 N values of the
 // storage scalar type (adjoint tape)
 // keep_sums (fused density): leave the tile sums in rho_next for k_mu_march<…, FIX>
-hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout = nullptr, bool keep_sums = false);
+// first / last: the step starts / ends a run (the populations are the state outside one)
+hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout = nullptr, bool keep_sums = false, bool first = true,
+                          bool last = true);
 hipError_t launch_macro(cpmp_ctx *c);
-hipError_t launch_step(cpmp_ctx *c, bool want_mv);
-// nsteps whole steps (MV on the last), advancing c->step
-hipError_t launch_steps(cpmp_ctx *c, int nsteps);
+// nsteps whole steps (MV on the last if wanted)
+hipError_t launch_steps(cpmp_ctx *c, int nsteps, bool want_mv = true);
 hipError_t launch_init_reference(cpmp_ctx *c, double radius, double width, double rg, double rl, double solid);
 hipError_t launch_init_splash(cpmp_ctx *c, double radius, double width, double film, double rg, double rl);
 hipError_t launch_init_spheres(cpmp_ctx *c, const cpmp_init_desc *d);

@@ -1581,7 +1581,7 @@ int march_chunk(int nx, int ny, int nz, int form) {
         if ((nx + c - 1) / c * tiles >= 1024) return c;
     return 2;
 }
-bool density_fused(const cpmp_ctx *c) { return c->rbuf && !c->collide_v1; }
+bool density_fused(const cpmp_ctx *c) { return c->rbuf && !c->collide_v1 && !c->moments; }
 
 // FP64 lattices with fewer than 2048 march workgroups of 2 planes: the per-node
 // collide (2 waves per SIMD, no LDS ring) measured 8 % faster per step at 64^3 and
@@ -1643,7 +1643,19 @@ hipError_t launch_mu(cpmp_ctx *c, void *rho_copy) {
     });
 }
 
-hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool keep_sums) {
+bool moment_path(const cpmp_params &p, const DevParams &d, bool fuse_off, bool covered) {
+    const char *e = std::getenv("CPMP_COLLIDE");
+    if (!d.unit_rates || p.form == CPMP_FORM_FP16 || (e && std::strcmp(e, "v1") == 0) || (fuse_off && covered)) return false;
+    return d.N >= 100000 || (e && std::strcmp(e, "march") == 0) || std::getenv("CPMP_XC");
+}
+
+hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool keep_sums, bool first, bool last) {
+    if (c->moments) {
+        const hipError_t e = launch_moment_step(c, first, last, want_mv, uout_v);
+        c->cur ^= 1;
+        std::swap(c->rho, c->rho_next);
+        return e;
+    }
     const bool rs = density_fused(c);
     const hipError_t e = dispatch(c->form, [&](auto fm) {
         using TF = typename decltype(fm)::TF;
@@ -1676,7 +1688,6 @@ hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool keep_sum
         } else {
             const int ntz = (c->p.nz + MTZ - 1) / MTZ, nty = (c->p.ny + MTY - 1) / MTY, nch = (c->p.nx + c->dp.xc - 1) / c->dp.xc;
             const dim3 grid((unsigned)(ntz * nty * nch));
-            constexpr bool can_rs = true;
             // MV, RS and the unit-rate specialisation as template arguments
             // NW: no solid layers (lo = hi = 0), the bounce-back selects compile away
             const bool nw = c->dp.lo == 0 && c->dp.hi == 0;
@@ -1705,11 +1716,16 @@ hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool keep_sum
             };
             using T1 = std::true_type;
             using F0 = std::false_type;
-            using RSB = std::integral_constant<bool, can_rs>;
             const bool ur = c->dp.unit_rates != 0;
-            if (can_rs && rs) {
-                if (want_mv) { if (ur) go(T1{}, RSB{}, T1{}); else go(T1{}, RSB{}, F0{}); }
-                else { if (ur) go(F0{}, RSB{}, T1{}); else go(F0{}, RSB{}, F0{}); }
+            // FP64 storage sums the density here with general rates only (the unit-rate
+            // lattices take the moments)
+            if (rs) {
+                if constexpr (std::is_same<TF, double>::value) {
+                    if (want_mv) go(T1{}, T1{}, F0{}); else go(F0{}, T1{}, F0{});
+                } else {
+                    if (want_mv) { if (ur) go(T1{}, T1{}, T1{}); else go(T1{}, T1{}, F0{}); }
+                    else { if (ur) go(F0{}, T1{}, T1{}); else go(F0{}, T1{}, F0{}); }
+                }
             } else {
                 if (want_mv) { if (ur) go(T1{}, F0{}, T1{}); else go(T1{}, F0{}, F0{}); }
                 else { if (ur) go(F0{}, F0{}, T1{}); else go(F0{}, F0{}, F0{}); }
@@ -1725,6 +1741,7 @@ hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool keep_sum
 }
 
 hipError_t launch_macro(cpmp_ctx *c) {
+    if (c->moments) return hipSuccess;   // the moment step leaves the density complete
     if (density_fused(c)) {   // summed by the collide kernel; add the tile and chunk borders
         return dispatch(c->form, [&](auto fm) {
             using TS = typename decltype(fm)::TS;
@@ -1747,14 +1764,6 @@ hipError_t launch_macro(cpmp_ctx *c) {
     });
     if (c->rho_next) std::swap(c->rho, c->rho_next);
     return e;
-}
-
-hipError_t launch_step(cpmp_ctx *c, bool want_mv) {
-    hipError_t e;
-    if ((e = launch_wall(c)) != hipSuccess) return e;
-    if ((e = launch_mu(c)) != hipSuccess) return e;
-    if ((e = launch_collide(c, want_mv)) != hipSuccess) return e;
-    return launch_macro(c);
 }
 
 // Periodic FP32 lattices with the density summed by the collide kernel: within a
@@ -1784,7 +1793,7 @@ static hipError_t launch_mu_fix(cpmp_ctx *c) {
     return hipGetLastError();
 }
 
-hipError_t launch_steps(cpmp_ctx *c, int nsteps) {
+hipError_t launch_steps(cpmp_ctx *c, int nsteps, bool want_mv) {
     const bool defer = fix_deferrable(c);
     hipError_t e;
     for (int n = 0; n < nsteps; ++n) {
@@ -1798,10 +1807,9 @@ hipError_t launch_steps(cpmp_ctx *c, int nsteps) {
         if (defer && !last) {
             if ((e = launch_collide(c, false, nullptr, true)) != hipSuccess) return e;
         } else {
-            if ((e = launch_collide(c, last)) != hipSuccess) return e;
+            if ((e = launch_collide(c, last && want_mv, nullptr, false, n == 0, last)) != hipSuccess) return e;
             if ((e = launch_macro(c)) != hipSuccess) return e;
         }
-        ++c->step;
     }
     return hipSuccess;
 }

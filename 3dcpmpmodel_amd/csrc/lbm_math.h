@@ -182,8 +182,10 @@ CPMP_HD void momentum(const T f[Q], T &jx, T &jy, T &jz) {
 //   m* = m - S(m - Meq(rho,u)) + S Qp + [Meq(rho,u+F/rho) - Meq(rho,u)]
 //      = (I - S)(m - Meq(rho,u)) + Meq(rho,u+F/rho) + S Qp
 //   out = R m*
-// The bracket is M (Feq(rho,EV) - Feq(rho,u)), the exact-difference force term of
-// FluidCuda.cu:341, since M Feq(rho,v) = Meq(rho,v) for this basis.  u = j/rho with
+// with m = M f the moments of the pulled populations (of the unit_rate_row rows only
+// 3, 5 and 7 are read under UR).  The bracket is M (Feq(rho,EV) - Feq(rho,u)), the
+// exact-difference force term of FluidCuda.cu:341, since M Feq(rho,v) = Meq(rho,v) for
+// this basis.  u = j/rho with
 // j = (m3, m5, m7) and rho the stored density; it is returned in u[3].  Each row
 // is finished as soon as its equilibrium values are formed, which keeps the
 // number of live registers low.
@@ -212,9 +214,7 @@ CPMP_HD T recip(T x) {
 // G16..18 = 0.  Mass is conserved and the momentum gains F exactly.  u returns j/rho
 // in both forms.
 template <class T, bool UR = false, bool GUO = false>
-CPMP_HD void collide(const T f[Q], T rho, T Fx, T Fy, T Fz, const T *ts, const T *qp, T out[Q], T u[3]) {
-    T m[Q];
-    moments(f, m);
+CPMP_HD void collide_moments(const T m[Q], T rho, T Fx, T Fy, T Fz, const T *ts, const T *qp, T out[Q], T u[3]) {
     const T inv = recip(rho);
     const T ux = m[3] * inv, uy = m[5] * inv, uz = m[7] * inv;
     u[0] = ux; u[1] = uy; u[2] = uz;
@@ -277,6 +277,14 @@ CPMP_HD void collide(const T f[Q], T rho, T Fx, T Fy, T Fz, const T *ts, const T
 #pragma unroll
     for (int r = 16; r < Q; ++r) a[r] = UR ? T(0) : (T(1) - ts[r]) * m[r] * T(1.0 / n2(r));
     inverse_scaled<T, UR>(a, out);
+}
+
+// the same collision from the pulled populations
+template <class T, bool UR = false, bool GUO = false>
+CPMP_HD void collide(const T f[Q], T rho, T Fx, T Fy, T Fz, const T *ts, const T *qp, T out[Q], T u[3]) {
+    T m[Q];
+    moments(f, m);
+    collide_moments<T, UR, GUO>(m, rho, Fx, Fy, Fz, ts, qp, out, u);
 }
 
 // Qp of FluidCuda.cu:260-266 from the density gradient (K1, K2 tuning).

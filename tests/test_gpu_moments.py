@@ -1,0 +1,93 @@
+"""Runs of steps on 13 moments per node (k_moment_step) against the population kernels.
+
+The moments carry exactly what the collision reads at the reference's rates, so a run
+must agree with the one-thread-per-node population kernels (CPMP_COLLIDE=v1) to the
+rounding of its sums.  The sizes are the edges of the 12 x 32 (y, z) tiles and of the
+x chunks: one row or column more or less than a tile, a tile of a single column, fewer
+planes than the stencils reach, chunks of one plane and longer than the lattice, and
+the one-row lattices with their own tile of 192 columns."""
+import os
+
+import numpy as np
+import pytest
+
+import gpu_cases as gc
+
+pytestmark = pytest.mark.gpu
+
+# dims, chunk, walls, options
+CASES = [
+    ((9, 12, 32), 4, 0, {}),
+    ((8, 13, 33), 3, 3, {}),                    # a tile of one row, a tile of one column
+    ((7, 11, 31), 7, 0, {}),                    # below one tile; nx below 8 (general wrap)
+    ((1, 24, 64), 1, 0, {}),
+    ((5, 25, 65), 2, 0, dict(lap_points=7)),
+    ((10, 2, 40), 10, 3, dict(wall_scheme=0)),
+    ((16, 14, 20), 64, 3, dict(wall_scheme=2)),
+    ((12, 13, 34), 5, 3, dict(K1=0.003, K2=-0.003)),
+    ((12, 23, 24), 5, 3, dict(forcing=1)),
+    ((12, 13, 34), 5, 0, dict(forcing=1, K1=0.003, K2=-0.003)),
+    ((20, 1, 191), 6, 3, {}),
+    ((6, 1, 193), 1, 0, {}),
+    ((11, 1, 385), 4, 3, dict(forcing=1)),
+]
+
+
+def lattice(cpmp, monkeypatch, case, form, collide):
+    dims, xc, nwall, opts = case
+    monkeypatch.setenv("CPMP_COLLIDE", collide)
+    monkeypatch.setenv("CPMP_XC", str(xc))
+    g = cpmp.Lattice(cpmp.make_params(*dims, eos="VDW", tr=0.8, nwall=nwall, form=form, **opts))
+    monkeypatch.delenv("CPMP_COLLIDE")
+    monkeypatch.delenv("CPMP_XC")
+    if nwall:
+        g.set_wall_mu(0.002, 0.01)
+    rng = np.random.default_rng(7)
+    nx, ny, nz = dims
+    rho = 3.5 + 0.3 * rng.standard_normal(dims)
+    rho[:, :, :nwall] = rho[:, :, nz - nwall:] = 0
+    g.init_from_rho(rho.ravel())
+    return g
+
+
+@pytest.mark.parametrize("form,tol", [("fp64", 1e-12), ("fp32", 1e-5), ("fp32a", 1e-5)])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[0])))
+def test_moment_runs_match_the_population_kernels(cpmp, monkeypatch, case, form, tol):
+    """7 steps from rough densities (every node differs from its neighbours, so a value
+    taken from a wrong node shows at once).  A step sums 19 values and the moments once
+    more, some 40 roundings of at most the largest population: 7 * 40 * 2^-53 = 3e-14
+    (FP64) and 1.7e-5 / 2 (FP32) relative to the density, and smaller in practice."""
+    a = lattice(cpmp, monkeypatch, case, form, "march")
+    b = lattice(cpmp, monkeypatch, case, form, "v1")
+    a.step(7)
+    b.step(7)
+    fluid = a.get("type") == 1
+    for field in ("rho", "f", "mv", "mu"):
+        x, y = a.get(field).reshape(-1, fluid.size)[:, fluid], b.get(field).reshape(-1, fluid.size)[:, fluid]
+        scale = np.max(np.abs(b.get("rho"))) if field in ("rho", "f") else max(np.max(np.abs(y)), 0.1)
+        err = np.max(np.abs(x - y)) / scale
+        print(f"[moments] {case[0]} {form} {field}: {err:.2e}", flush=True)
+        assert err < tol, field
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("form", ["fp64", "fp32", "fp32a"])
+@pytest.mark.parametrize("case", [CASES[1], CASES[7], CASES[8], CASES[10]], ids=lambda c: "x".join(map(str, c[0])))
+def test_moment_runs_split_into_calls_are_bitwise_the_same(cpmp, monkeypatch, tmp_path, case, form):
+    """the populations between calls lose nothing: one call of 6 steps, and calls of
+    1 + 2 + 3 steps with a checkpoint taken into another lattice in between"""
+    a = lattice(cpmp, monkeypatch, case, form, "march")
+    b = lattice(cpmp, monkeypatch, case, form, "march")
+    c = lattice(cpmp, monkeypatch, case, form, "march")
+    a.step(6)
+    b.step(1)
+    b.step(2)
+    path = str(tmp_path / "split.ckp")
+    b.checkpoint_save(path)
+    c.checkpoint_load(path)
+    c.step(3)
+    for field in ("rho", "mu", "f", "mv"):
+        assert np.array_equal(a.get(field), c.get(field)), field
+    for g in (a, b, c):
+        g.close()
