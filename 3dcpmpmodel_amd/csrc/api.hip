@@ -75,7 +75,7 @@ void fill_devparams(cpmp_ctx *c) {
     d.N = (long long)p.nx * p.ny * p.nz;
     d.eos = p.eos; d.mu_form = p.mu_form; d.lap_points = p.lap_points; d.wall_scheme = p.wall_scheme;
     d.qp_on = (p.K1 != 0.0 || p.K2 != 0.0) ? 1 : 0;
-    d.A = p.A; d.B = p.B; d.T = p.T; d.K2s = p.K * p.K; d.Ka = p.Ka; d.K1 = p.K1; d.K2 = p.K2;
+    d.A = p.A; d.B = p.B; d.T = p.T; d.K2s = p.K * p.K; d.AoB = p.A / p.B; d.AoPr = p.A / (2 * kSqrt2 * p.B); d.Ka = p.Ka; d.K1 = p.K1; d.K2 = p.K2;
     for (int q = 0; q < 19; ++q) { d.ts[q] = p.Ts[q]; d.tsf[q] = (float)p.Ts[q]; }
     d.unit_rates = 1;
     for (int q = 0; q < 19; ++q)

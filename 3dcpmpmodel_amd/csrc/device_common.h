@@ -98,6 +98,46 @@ __device__ __forceinline__ void wrap7(const DevParams &P, const Coord &c, int *x
     }
 }
 
+// FP64 reciprocal: the hardware estimate and two Newton steps (within 1 ulp; finite
+// non-zero x)
+__device__ __forceinline__ double recip64(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
+// FP64 natural logarithm within 1 ulp.  x = 2^k m with m in [sqrt(1/2), sqrt(2)),
+// f = m - 1 (exact), s = f / (2 + f):  ln m = 2 atanh(s) = 2 s + s R,
+// R = 2 s^2 (1/3 + s^2/5 + s^4/7 + ..), |s| <= 0.172, so the series to s^20 / 23 leaves
+// 3e-18; written as f - (f^2/2 - s (f^2/2 + R)), where only small terms carry the rounding
+// of s.  The device library's log costs about twice the instructions.
+__device__ __forceinline__ double ln64(double x) {
+    if (!__builtin_amdgcn_class(x, 0x180))   // not positive, finite and non-zero
+        return x == 0.0 ? -__builtin_inf() : x > 0.0 ? x : __builtin_nan("");
+    double m = __builtin_amdgcn_frexp_mant(x);
+    int k = __builtin_amdgcn_frexp_exp(x);
+    const bool low = m < 0.70710678118654752440;
+    m = low ? 2.0 * m : m;
+    k = low ? k - 1 : k;
+    const double f = m - 1.0, den = 2.0 + f, s = f * recip64(den), z = s * s;
+    double r = 2.0 / 23;
+    r = fma(r, z, 2.0 / 21);
+    r = fma(r, z, 2.0 / 19);
+    r = fma(r, z, 2.0 / 17);
+    r = fma(r, z, 2.0 / 15);
+    r = fma(r, z, 2.0 / 13);
+    r = fma(r, z, 2.0 / 11);
+    r = fma(r, z, 2.0 / 9);
+    r = fma(r, z, 2.0 / 7);
+    r = fma(r, z, 2.0 / 5);
+    r = fma(r, z, 2.0 / 3);
+    r *= z;
+    const double h = 0.5 * f * f, kd = (double)k;
+    // k ln 2 in two parts: the high one has 32 significant bits, so its product is exact
+    const double hi = 0x1.62e42fee00000p-1, lo = 0x1.a39ef35793c76p-33;
+    return kd * hi - ((h - fma(s, h + r, kd * lo)) - f);
+}
+
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

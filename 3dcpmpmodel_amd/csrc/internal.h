@@ -19,6 +19,7 @@ struct DevParams {
     int eos, mu_form, lap_points, wall_scheme;
     int qp_on;                  // K1 or K2 non-zero
     double A, B, T, K2s, Ka;    // K2s = K*K
+    double AoB, AoPr;           // A / B, A / (2 sqrt(2) B)
     double K1, K2;
     double ts[19];
     float tsf[19];              // ts in FP32 for the FP32 arithmetic forms

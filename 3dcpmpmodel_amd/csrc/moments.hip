@@ -211,16 +211,16 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 && !IN_P ? 4 : 2) k_mo
         eoff[h] = (unsigned)((TL::flat ? 0 : wrapc(y0 - 4 + ey, P.ny)) * P.nz + wrapc(z0 - 4 + ez, P.nz));
     }
     TC er[TL::HE], em[TL::HE];
-    auto fetch_ring = [&](int x) {
+    auto fetch_plane = [&](int x, TC (&r)[TL::HE], TC (&m)[TL::HE]) {
         const size_t b = (size_t)wrap_x(x) * pl;
         const TS *rp = A.rho + b, *mp = A.mu + b;
 #pragma unroll
-        for (int h = 0; h < TL::HE; ++h) { er[h] = (TC)*lane_at(rp, eoff[h]); em[h] = (TC)*lane_at(mp, eoff[h]); }
+        for (int h = 0; h < TL::HE; ++h) { r[h] = (TC)*lane_at(rp, eoff[h]); m[h] = (TC)*lane_at(mp, eoff[h]); }
     };
-    auto store_ring = [&](int slot) {
+    auto store_plane = [&](int slot, const TC (&r)[TL::HE], const TC (&m)[TL::HE]) {
 #pragma unroll
         for (int h = 0; h < TL::HE; ++h)
-            if ((h + 1) * TL::NT <= TL::EP || tid + h * TL::NT < TL::EP) s_rm[slot][tid + h * TL::NT] = Pair<TC>{er[h], em[h]};
+            if ((h + 1) * TL::NT <= TL::EP || tid + h * TL::NT < TL::EP) s_rm[slot][tid + h * TL::NT] = Pair<TC>{r[h], m[h]};
     };
 
     // the state before the step at this thread's node of plane x
@@ -248,12 +248,15 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 && !IN_P ? 4 : 2) k_mo
         }
     };
 
-    for (int k = 0; k < 7; ++k) {
-        fetch_ring(xa - 4 + k);
-        store_ring(k);
+    {   // the first seven planes, all loads in flight at once
+        TC r7[7][TL::HE], m7[7][TL::HE];
+#pragma unroll
+        for (int k = 0; k < 7; ++k) fetch_plane(xa - 4 + k, r7[k], m7[k]);
+        fetch_state(xa - 1);
+#pragma unroll
+        for (int k = 0; k < 7; ++k) store_plane(k, r7[k], m7[k]);
     }
-    fetch_ring(xa + 3);
-    fetch_state(xa - 1);
+    fetch_plane(xa + 3, er, em);
     int s0 = 0;   // ring slot of plane x - 3
     const int one = z0 == zlast ? kMom * TL::TY : TL::NT;
     // a finished plane's edge columns, from LDS to memory
@@ -337,8 +340,8 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 && !IN_P ? 4 : 2) k_mo
             }
         }
         __syncthreads();                       // mailbox of plane x posted, plane x - 3 no longer read
-        store_ring(s0);                        // plane x + 4
-        fetch_ring(x + 5);
+        store_plane(s0, er, em);               // plane x + 4
+        fetch_plane(x + 5, er, em);
         s0 = s0 == 6 ? 0 : s0 + 1;
         if (inner) {
             // what arrives along q: the neighbour's value, or the node's own along opp(q)
