@@ -795,6 +795,7 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
             return e != hipSuccess ? e : hipMemcpyAsync(dst + fbytes, c->rho, rbytes, hipMemcpyDeviceToDevice, c->stream);
         };
         auto restore = [&](const char *src) -> hipError_t {
+            c->mom_at = 0;   // the moments are not those of the restored populations
             hipError_t e = hipMemcpyAsync(c->f[c->cur], src, fbytes, hipMemcpyDeviceToDevice, c->stream);
             return e != hipSuccess ? e : hipMemcpyAsync(c->rho, src + fbytes, rbytes, hipMemcpyDeviceToDevice, c->stream);
         };
@@ -805,7 +806,7 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
                 hipError_t e;
                 if ((e = launch_wall(c)) != hipSuccess) return e;
                 if ((e = launch_mu(c, tr)) != hipSuccess) return e;   // also copies rho (after the wall fill) to tr
-                if ((e = launch_collide(c, false, tr + N * sb, false, k == 0, k == L - 1)) != hipSuccess) return e;
+                if ((e = launch_collide(c, false, tr + N * sb, k == L - 1)) != hipSuccess) return e;
                 if ((e = launch_macro(c)) != hipSuccess) return e;
             }
             return hipSuccess;
@@ -940,6 +941,7 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
     if (g_lo) AHIP(hipMemcpyAsync(g_lo, gl, NXY * sizeof(double), hipMemcpyDeviceToHost, s));
     if (g_hi) AHIP(hipMemcpyAsync(g_hi, gh, NXY * sizeof(double), hipMemcpyDeviceToHost, s));
     // leave the context at the end of the forward run
+    c->mom_at = 0;
     {
         const hipError_t e = hipMemcpyAsync(c->f[c->cur], fin, fbytes, hipMemcpyDeviceToDevice, s);
         AHIP(e);

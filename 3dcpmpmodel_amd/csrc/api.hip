@@ -53,20 +53,6 @@ hipError_t sync_reference_density(cpmp_ctx *c) {
 int pop_size(int form) { return fp64_storage(form) ? 8 : (form == CPMP_FORM_FP32 ? 4 : 2); }
 int scal_size(int form) { return fp64_storage(form) ? 8 : 4; }
 
-// interface runs of the chemical-potential march (FP32 storage forms): 64 * xc
-// slots per wave, MT / 64 waves per workgroup
-size_t band_slots(const cpmp_ctx *c) {
-    const size_t xc = (size_t)c->dp.xc;
-    const size_t blocks = (size_t)((c->p.nz + kTileZ - 1) / kTileZ) * ((c->p.ny + kTileY - 1) / kTileY) * ((c->p.nx + xc - 1) / xc);
-    return blocks * kTileY * kTileZ * xc;
-}
-// overflow descriptors: a run of n entries posts ceil((n - kBandWave) / kBandDesc) <=
-// n / kBandDesc + 1, so slots / kBandDesc + (runs) bound their number
-size_t band_desc_slots(const cpmp_ctx *c) {
-    const size_t runs = band_slots(c) / (64 * (size_t)c->dp.xc);
-    return band_slots(c) / kBandDesc + runs + 1;
-}
-
 void fill_devparams(cpmp_ctx *c) {
     const cpmp_params &p = c->p;
     DevParams &d = c->dp;
@@ -290,12 +276,14 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
     size_t ring_elems = 0, chunk_elems = 0;
     const bool fuse_off = fuse && std::strcmp(fuse, "0") == 0;
     const bool covered = fuse_geometry(p->nx, p->ny, p->nz, c->dp.xc, &ring_elems, &chunk_elems);
-    c->moments = moment_path(*p, c->dp, fuse_off, covered);
+    const size_t mset = moment_bytes(p->nx, p->ny, p->nz, p->form);
+    c->moments = mset <= popset && moment_path(*p, c->dp, fuse_off, covered);
     if (c->moments) {
         c->collide_v1 = false;
         c->step_chunk = moment_chunk(p->nx, p->ny, p->nz, p->form);
         if (hipMalloc(&c->rho_next, c->N * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "next rho");
-        c->fuse_bytes = (size_t)c->N * c->scal_bytes;
+        if (hipMalloc(&c->mom, mset) != hipSuccess) return fail(CPMP_ENOMEM, "moments");
+        c->fuse_bytes = (size_t)c->N * c->scal_bytes + mset;
     }
     // the population march sums the density inside the collide where the tiles cover the
     // lattice (not the one-thread-per-node collide of small FP64 lattices).  The adjoint of
@@ -304,7 +292,7 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
         if (!c->rho_next && hipMalloc(&c->rho_next, c->N * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "next rho");
         if (hipMalloc(&c->rbuf, ring_elems * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "tile rings");
         if (hipMalloc(&c->cbuf, chunk_elems * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "chunk planes");
-        c->fuse_bytes = ((size_t)c->N + ring_elems + chunk_elems) * c->scal_bytes;
+        c->fuse_bytes = ((size_t)c->N + ring_elems + chunk_elems) * c->scal_bytes + (c->mom ? mset : 0);
     }
     if (covered && !fuse_off && !c->collide_v1) {   // populations tile-contiguous (pop_site)
         c->dp.tiled = 1;
@@ -317,15 +305,6 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
         if (hipMalloc(&c->rho_next, c->N * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "previous rho");
         c->fuse_bytes = (size_t)c->N * c->scal_bytes;
     }
-    if (!fp64_storage(c->form)) {
-        if (hipMalloc((void **)&c->band, band_slots(c) * sizeof(uint4)) != hipSuccess)
-            return fail(CPMP_ENOMEM, "interface runs");
-        // descriptors, then the two counters
-        if (hipMalloc((void **)&c->band_ovf, (band_desc_slots(c) + 1) * sizeof(uint2)) != hipSuccess)
-            return fail(CPMP_ENOMEM, "interface overflow");
-        c->band_cnt = (unsigned *)(c->band_ovf + band_desc_slots(c));
-        c->band_cap = (unsigned)band_desc_slots(c);
-    }
     if (hipMalloc((void **)&c->mv, 3 * c->N * sizeof(double)) != hipSuccess) return fail(CPMP_ENOMEM, "MV");
     if (hipMalloc((void **)&c->mu_w, 2 * c->NXY * sizeof(double)) != hipSuccess) return fail(CPMP_ENOMEM, "wall mu");
     if (hipMalloc((void **)&c->red, reduce_scratch_doubles() * sizeof(double)) != hipSuccess) return fail(CPMP_ENOMEM, "reduce");
@@ -334,7 +313,6 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
         hipMemsetAsync(c->rho, 0, c->N * c->scal_bytes, c->stream) != hipSuccess ||
         hipMemsetAsync(c->mu, 0, c->N * c->scal_bytes, c->stream) != hipSuccess ||
         (c->rho_next && hipMemsetAsync(c->rho_next, 0, c->N * c->scal_bytes, c->stream) != hipSuccess) ||
-        (c->band_cnt && hipMemsetAsync(c->band_cnt, 0, 2 * sizeof(unsigned), c->stream) != hipSuccess) ||
         hipMemsetAsync(c->mv, 0, 3 * c->N * sizeof(double), c->stream) != hipSuccess ||
         hipMemsetAsync(c->mu_w, 0, 2 * c->NXY * sizeof(double), c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
@@ -346,8 +324,8 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
 int cpmp_destroy(cpmp_ctx *c) {
     if (!c) return CPMP_OK;
     if (c->stream) { hipSetDevice(c->p.device); hipStreamSynchronize(c->stream); }
-    for (void *ptr : {c->f[0], c->f[1], c->rho, c->rho_next, c->rbuf, c->cbuf, c->mu, (void *)c->band,
-                      (void *)c->band_ovf, (void *)c->mv, (void *)c->mu_w, (void *)c->red, (void *)c->staging})
+    for (void *ptr : {c->f[0], c->f[1], c->rho, c->rho_next, c->rbuf, c->cbuf, c->mom, c->mu, (void *)c->mv, (void *)c->mu_w,
+                      (void *)c->red, (void *)c->staging})
         if (ptr) hipFree(ptr);
     if (c->timers) {
         for (auto &e : c->timers->ev) if (e) hipEventDestroy(e);
@@ -367,8 +345,7 @@ int cpmp_get_params(cpmp_ctx *c, cpmp_params *out) {
 int cpmp_memory(cpmp_ctx *c, int64_t *bytes) {
     if (!valid_ctx(c) || !bytes) return set_error(CPMP_EINVAL, "bad context or output");
     *bytes = (int64_t)(2 * (size_t)c->N * 19 * c->pop_bytes + 2 * c->N * c->scal_bytes + 4 * c->N * sizeof(double)
-                       + 2 * c->NXY * sizeof(double) + reduce_scratch_doubles() * sizeof(double) + c->fuse_bytes
-                       + (c->band ? band_slots(c) * sizeof(uint4) + (band_desc_slots(c) + 1) * sizeof(uint2) : 0));
+                       + 2 * c->NXY * sizeof(double) + reduce_scratch_doubles() * sizeof(double) + c->fuse_bytes);
     return CPMP_OK;
 }
 
@@ -383,6 +360,7 @@ int cpmp_init_reference(cpmp_ctx *c, double radius, double width, double rg, dou
     HIPCHK(hipStreamSynchronize(c->stream));
     c->step = 0;
     c->mv_valid = false;
+    c->mom_at = 0;
     return CPMP_OK;
 }
 
@@ -396,6 +374,7 @@ int cpmp_init_splash(cpmp_ctx *c, double radius, double width, double film_z, do
     HIPCHK(hipStreamSynchronize(c->stream));
     c->step = 0;
     c->mv_valid = false;
+    c->mom_at = 0;
     return CPMP_OK;
 }
 
@@ -410,6 +389,7 @@ int cpmp_init_spheres(cpmp_ctx *c, const cpmp_init_desc *d) {
     HIPCHK(hipStreamSynchronize(c->stream));
     c->step = 0;
     c->mv_valid = false;
+    c->mom_at = 0;
     return CPMP_OK;
 }
 
@@ -424,6 +404,7 @@ int cpmp_init_from_rho(cpmp_ctx *c, const double *rho) {
     HIPCHK(hipStreamSynchronize(c->stream));
     c->step = 0;
     c->mv_valid = false;
+    c->mom_at = 0;
     return CPMP_OK;
 }
 
@@ -524,6 +505,7 @@ int cpmp_set_field(cpmp_ctx *c, int field, const double *host) {
         HIPCHK(launch_scalar_from_double(c, c->staging, field == CPMP_FIELD_RHO ? c->rho : c->mu));
         break;
     case CPMP_FIELD_F:
+        c->mom_at = 0;
         for (int q = 0; q < 19; ++q) {
             HIPCHK(hipMemcpyAsync(c->staging, host + (size_t)q * c->N, nb, hipMemcpyHostToDevice, c->stream));
             HIPCHK(launch_pop_from_double(c, q, c->staging, c->f[c->cur]));
@@ -583,6 +565,7 @@ int cpmp_checkpoint_save(cpmp_ctx *c, const char *path) {
     // populations in the reference node order whatever the device layout
     const void *pops = c->f[c->cur];
     if (c->dp.tiled) {
+        if (c->mom_at == 2) c->mom_at = 0;   // the other set is the scratch of the copy
         HIPCHK(launch_pop_relayout(c, c->f[c->cur], c->f[c->cur ^ 1], false));
         pops = c->f[c->cur ^ 1];
     }
@@ -628,6 +611,7 @@ int cpmp_checkpoint_load(cpmp_ctx *c, const char *path) {
     std::fclose(fp);
     if (!ok) return set_error(CPMP_EIO, "%s is truncated", path);
     HIPCHK(hipSetDevice(c->p.device));
+    c->mom_at = 0;
     if (c->dp.tiled) {
         HIPCHK(hipMemcpyAsync(c->f[c->cur ^ 1], buf.data(), popset, hipMemcpyHostToDevice, c->stream));
         HIPCHK(launch_pop_relayout(c, c->f[c->cur ^ 1], c->f[c->cur], true));
@@ -687,7 +671,7 @@ int cpmp_kernel_times(cpmp_ctx *c, int nsteps, double *ms, int *launches) {
         HIPCHK(launch_mu(c));
         HIPCHK(hipEventRecord(ev[3], c->stream));
         HIPCHK(hipEventRecord(ev[4], c->stream));
-        HIPCHK(launch_collide(c, n == nsteps - 1, nullptr, false, n == 0, n == nsteps - 1));
+        HIPCHK(launch_collide(c, n == nsteps - 1, nullptr, n == nsteps - 1));
         HIPCHK(hipEventRecord(ev[5], c->stream));
         HIPCHK(hipEventRecord(ev[6], c->stream));
         HIPCHK(launch_macro(c));

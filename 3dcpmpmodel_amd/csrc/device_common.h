@@ -6,6 +6,8 @@
 #include "internal.h"
 #include "lbm_math.h"
 
+#include <type_traits>
+
 namespace cpmp {
 
 constexpr int TPB = 256;
@@ -96,6 +98,21 @@ __device__ __forceinline__ void wrap7(const DevParams &P, const Coord &c, int *x
         ys[s] = wrap_off(c.y, s - 3, P.ny);
         zs[s] = wrap_off(c.z, s - 3, P.nz);
     }
+}
+
+// Address `bytes` past a base that is uniform over the wave: the offset stays in 32 bits (a
+// plane of at most 2^31 / 19 values of 8 bytes fits), so the access takes the scalar-base
+// form and no 64-bit address is kept per lane.
+template <class T>
+__device__ __forceinline__ T *lane_bytes(T *base, unsigned bytes) {
+    using C = std::conditional_t<std::is_const<T>::value, const char, char>;
+    return (T *)((C *)base + bytes);
+}
+// An empty asm makes a loop-invariant offset a value of this pass of the loop: hoisted out
+// of the loop it would be kept zero-extended in two registers.
+__device__ __forceinline__ unsigned in_loop(unsigned v) {
+    asm volatile("" : "+v"(v));
+    return v;
 }
 
 // FP64 reciprocal: the hardware estimate and two Newton steps (within 1 ulp; finite

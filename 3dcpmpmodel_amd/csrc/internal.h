@@ -60,20 +60,13 @@ struct cpmp_ctx {
     // FP32 storage forms on exactly tiled lattices: density summed by the collide
     // kernel into rho_next, tile rings and chunk partial planes for the fix-up pass
     void *rho_next = nullptr, *rbuf = nullptr, *cbuf = nullptr;
-    // FP32 storage forms: per wave of the chemical-potential march, a run of 64 * xc
-    // slots (node, density, Laplacian term) for the interface nodes it finishes in FP64
-    uint4 *band = nullptr;
-    // the entries of a run beyond the first kBandWave: descriptors (first slot, count of
-    // at most kBandDesc) that k_band_overflow finishes after the march, and two counters
-    // of posted descriptors used by alternate launches (band_par), each cleared by the
-    // overflow kernel of the launch before its use
-    uint2 *band_ovf = nullptr;
-    unsigned *band_cnt = nullptr;
-    unsigned band_cap = 0;      // descriptor slots
-    int band_par = 0;
     bool collide_v1 = false;    // one-thread-per-node collide (node_collide)
     bool moments = false;       // runs of steps carry 13 moments per node (moment_path)
     int step_chunk = 0;         // x planes per workgroup of the moment step
+    // a moment set; the population set that is not current holds the other.  mom_at: which
+    // one holds the moments of the current populations (0 none, 1 mom, 2 the population set)
+    void *mom = nullptr;
+    int mom_at = 0;
     size_t fuse_bytes = 0;
     double *mv = nullptr;       // 3*N, MV of the last step
     double *mu_w = nullptr;     // 2*NXY: bottom then top
@@ -96,8 +89,6 @@ bool density_fused(const cpmp_ctx *c);
 bool fuse_geometry(int nx, int ny, int nz, int xc, size_t *ring_elems, size_t *chunk_elems);
 // forms whose populations, rho and mu are stored in FP64 (FP64, FP32A)
 inline bool fp64_storage(int form) { return form == CPMP_FORM_FP64 || form == CPMP_FORM_FP32A; }
-constexpr unsigned kBandWave = 128;   // interface nodes a wave of the mu march finishes itself
-constexpr unsigned kBandDesc = 256;   // interface nodes per overflow descriptor (one workgroup)
 // x planes per march workgroup for a lattice and storage form (CPMP_XC overrides)
 int march_chunk(int nx, int ny, int nz, int form);
 // the one-thread-per-node collide instead of the x march (CPMP_COLLIDE=v1 / march
@@ -115,19 +106,20 @@ bool node_collide(int nx, int ny, int nz, int form);
 bool moment_path(const cpmp_params &p, const DevParams &d, bool fuse_off, bool covered);
 constexpr int kMomentFields = 12;
 int moment_chunk(int nx, int ny, int nz, int form);
-// one collide and stream step from the current set into the other: populations or
-// moments in and out; rho_next receives the new density of the fluid nodes
-hipError_t launch_moment_step(cpmp_ctx *c, bool in_pops, bool out_pops, bool want_mv, void *uout);
+// bytes of a moment set (which has to fit a population set)
+size_t moment_bytes(int nx, int ny, int nz, int form);
+// one collide and stream step, from the moments if they are current (c->mom_at), else from
+// the populations, to moments and (out_pops) populations; rho_next receives the new
+// density of the fluid nodes
+hipError_t launch_moment_step(cpmp_ctx *c, bool out_pops, bool want_mv, void *uout);
 constexpr int kTileY = 8, kTileZ = 32;   // in-plane tile of the march kernels and of tiled population storage
 constexpr int kWallTile = 16;             // columns per edge of the wall-fill tiles (16 x 16 workgroups)
 // copy one population set between the device layout and the reference node order
 hipError_t launch_pop_relayout(cpmp_ctx *c, const void *src, void *dst, bool to_device_layout);
 // uout (when given): u, grad mu, grad rho of every node, 9 N values of the
 // storage scalar type (adjoint tape)
-// keep_sums (fused density): leave the tile sums in rho_next for k_mu_march<…, FIX>
-// first / last: the step starts / ends a run (the populations are the state outside one)
-hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout = nullptr, bool keep_sums = false, bool first = true,
-                          bool last = true);
+// last: the step ends a run (outside a run the populations are the state)
+hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout = nullptr, bool last = true);
 hipError_t launch_macro(cpmp_ctx *c);
 // nsteps whole steps (MV on the last if wanted)
 hipError_t launch_steps(cpmp_ctx *c, int nsteps, bool want_mv = true);

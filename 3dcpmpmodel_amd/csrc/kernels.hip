@@ -181,192 +181,6 @@ __global__ void __launch_bounds__(kWallTile * kWallTile) k_wall_tile(const DevPa
 }
 
 // ---------------------------------------------------------------------------
-// Chemical potential (ChemPotential, FluidCuda.cu:444-463):
-//   mu = K^2 mu_eos(clamp(rho)) - Ka * Laplacian(rho).
-// FP64 form: all in FP64, the Laplacian as the reference writes it.
-// FP32 storage forms (mu is stored in FP32): the Laplacian is summed over the
-// differences rho_k - rho_0 (its coefficients sum to zero, so this is the same
-// operator, and the differences carry no cancellation), and mu_eos is evaluated
-// in FP32 with the hardware log2 and reciprocal (relative error of a few ulp,
-// below the FP32 rounding of the stored mu).
-
-// mu_eos in FP32 with v_log_f32 / v_rcp_f32; same closed forms as mu_eos_t
-__device__ __forceinline__ float ln_hw(float x) { return __builtin_amdgcn_logf(x) * 0.693147180559945f; }
-__device__ __forceinline__ float rcp_hw(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ float mu_eos_fast(int eos, int form, float A, float B, float T, float d) {
-    const float s2 = 1.41421356f;
-    const float bd = B * d, rom = rcp_hw(1.0f - bd);
-    if (form == 1 || eos == EOS_PRW || eos == EOS_PRM) {
-        return T * ln_hw(d * rom) - A * rcp_hw(s2 * 2.0f * B) * ln_hw((s2 - 1.0f + bd) * rcp_hw(s2 + 1.0f - bd))
-               + T * rom - A * d * rcp_hw(1.0f + bd * 2.0f - bd * bd);
-    }
-    if (eos == EOS_VDW) return T * ln_hw(d * rom) + T * rom - 2.0f * A * d;
-    if (eos == EOS_RKE || eos == EOS_RKS) {
-        const float op = 1.0f + bd;
-        return T * ln_hw(d * rom) + T * rom - A * rcp_hw(B) * ln_hw(op) - A * d * rcp_hw(op);
-    }
-    return T * (ln_hw(d) + (8.0f * bd - 9.0f * bd * bd + 3.0f * bd * bd * bd) * rom * rom * rom) - 2.0f * A * d;
-}
-
-// mu_eos in FP64 with ln64 and one reciprocal for all the quotients of an EOS (the closed
-// forms of mu_eos_t; for Peng-Robinson (sqrt2 - 1 + bd)(sqrt2 + 1 - bd) = 1 + 2 bd - bd^2,
-// so the quotient in its second logarithm is (sqrt2 - 1 + bd)^2 over the same denominator)
-__device__ __forceinline__ double mu_eos_fast(const DevParams &P, double d) {
-    if (d > 9.7) d = 9.7 + (d - 9.7) * recip64(1.0 + (d - 9.7) * 1.5);   // clamp_rho
-    const double A = P.A, T = P.T, bd = P.B * d, om = 1.0 - bd;
-    if (P.mu_form == 1 || P.eos == EOS_PRW || P.eos == EOS_PRM) {
-        const double q = 1.0 + 2.0 * bd - bd * bd, u = kSqrt2 - 1.0 + bd, r = recip64(om * q), rom = r * q, rq = r * om;
-        return T * ln64(d * rom) - P.AoPr * ln64(u * u * rq) + T * rom - A * d * rq;
-    }
-    if (P.eos == EOS_RKE || P.eos == EOS_RKS) {
-        const double op = 1.0 + bd, r = recip64(om * op), rom = r * op;
-        return T * ln64(d * rom) + T * rom - P.AoB * ln64(op) - A * d * (r * om);
-    }
-    const double rom = recip64(om);
-    if (P.eos == EOS_VDW) return T * ln64(d * rom) + T * rom - 2.0 * A * d;
-    return T * (ln64(d) + (8.0 * bd - 9.0 * bd * bd + 3.0 * bd * bd * bd) * (rom * rom * rom)) - 2.0 * A * d;
-}
-
-// FP32 mu of an interface node from its FP32 Laplacian term Ka * lap: the EOS part
-// in FP64, rounded once
-__device__ __forceinline__ float mu_band(const DevParams &P, float d, float kal) {
-    return (float)(P.K2s * mu_eos_fast(P, (double)d) - (double)kal);
-}
-__device__ __forceinline__ bool in_band(const DevParams &P, float d) { return d > P.band_lo && d < P.band_hi; }
-
-// mu at one fluid node; get(dx, dy, dz) returns rho at the offset node.  FP32:
-// interface nodes (in_band) get the EOS part in FP64 if EOS64, else the FP32 value;
-// kal_out (if given) receives the FP32 Laplacian term.
-template <class TS, bool EOS64 = true, class Get>
-__device__ __forceinline__ TS mu_node(const DevParams &P, Get get, float *kal_out = nullptr) {
-    if constexpr (sizeof(TS) == 8) {
-        const double d = get(0, 0, 0);
-        double kal;
-        if (P.lap_points == 7) {   // GradD7, Common.h:243-246
-            auto ax = [&](int ux, int uy, int uz) {
-                return 2 * get(-3 * ux, -3 * uy, -3 * uz) - 27 * get(-2 * ux, -2 * uy, -2 * uz)
-                       + 270 * get(-ux, -uy, -uz) + 270 * get(ux, uy, uz) - 27 * get(2 * ux, 2 * uy, 2 * uz)
-                       + 2 * get(3 * ux, 3 * uy, 3 * uz);
-            };
-            kal = P.Ka * (-d * 490 * 3 + ax(1, 0, 0) + ax(0, 1, 0) + ax(0, 0, 1)) / 180;
-        } else {                   // GradD5, Common.h:189-192
-            auto ax = [&](int ux, int uy, int uz) {
-                return -get(-2 * ux, -2 * uy, -2 * uz) + get(-ux, -uy, -uz) * 16 + get(ux, uy, uz) * 16
-                       - get(2 * ux, 2 * uy, 2 * uz);
-            };
-            kal = P.Ka * ((-d * 90 + ax(1, 0, 0) + ax(0, 1, 0) + ax(0, 0, 1)) / 12);
-        }
-        return P.K2s * mu_eos_fast(P, d) - kal;
-    } else {
-        const float d = get(0, 0, 0);
-        auto df = [&](int dx, int dy, int dz) { return (float)get(dx, dy, dz) - d; };
-        float lap;
-        if (P.lap_points == 7) {
-            auto ax = [&](int ux, int uy, int uz) {
-                return 2.0f * (df(-3 * ux, -3 * uy, -3 * uz) + df(3 * ux, 3 * uy, 3 * uz))
-                       - 27.0f * (df(-2 * ux, -2 * uy, -2 * uz) + df(2 * ux, 2 * uy, 2 * uz))
-                       + 270.0f * (df(-ux, -uy, -uz) + df(ux, uy, uz));
-            };
-            lap = (ax(1, 0, 0) + ax(0, 1, 0) + ax(0, 0, 1)) * (1.0f / 180.0f);
-        } else {
-            auto ax = [&](int ux, int uy, int uz) {
-                return 16.0f * (df(-ux, -uy, -uz) + df(ux, uy, uz)) - (df(-2 * ux, -2 * uy, -2 * uz) + df(2 * ux, 2 * uy, 2 * uz));
-            };
-            lap = (ax(1, 0, 0) + ax(0, 1, 0) + ax(0, 0, 1)) * (1.0f / 12.0f);
-        }
-        const float kal = (float)P.Ka * lap;
-        if (kal_out) *kal_out = kal;
-        if (EOS64 && in_band(P, d)) return mu_band(P, d, kal);
-        const float dc = d > 9.7f ? 9.7f + (d - 9.7f) * rcp_hw(1.0f + (d - 9.7f) * 1.5f) : d;   // clamp_rho
-        const float m = mu_eos_fast(P.eos, P.mu_form, (float)P.A, (float)P.B, (float)P.T, dc);
-        return (float)P.K2s * m - kal;
-    }
-}
-
-// The chemical-potential march finishes its interface nodes at the end: each wave
-// appends (node, density, Laplacian term) to its run as it goes (lanes in lane
-// order; count is the wave's running total, the same in every lane), then sets
-// their mu with the FP64 EOS part, 64 at a time.
-__device__ __forceinline__ void band_append(bool in, unsigned idx, float d, float kal, uint4 *run, unsigned &count) {
-    const unsigned long long m = __ballot(in);
-    const int lane = (int)__lane_id();
-    if (in) run[count + (unsigned)__popcll(m & ((1ull << lane) - 1ull))] =
-        make_uint4(idx, __float_as_uint(d), __float_as_uint(kal), 0u);
-    count += (unsigned)__popcll(m);
-}
-// A wave finishes the first kBandWave entries of its run; the rest (the interface
-// crosses some waves' 64 columns for most of their planes: up to ~1800 entries at 256^3
-// against a mean of ~70 per wave) goes to k_band_overflow in descriptors of kBandDesc
-// entries, so that no wave holds the end of the launch for tens of rounds of the FP64
-// EOS.  run_index: the run's first slot in the band array; ovf_cap: the descriptor
-// slots (never exceeded while each launch's counter starts at zero; past it a wave
-// marks its reserved slots empty and finishes all its entries itself).
-__device__ __forceinline__ void band_finish(const DevParams &P, const uint4 *run, unsigned count, float *mu,
-                                            unsigned run_index, uint2 *ovf, unsigned *ovf_cnt, unsigned ovf_cap) {
-    if (count == 0) return;   // uniform over the wave
-    __threadfence_block();    // entries written by other lanes are visible
-    if (count > kBandWave) {  // uniform
-        const unsigned extra = count - kBandWave, nd = (extra + kBandDesc - 1) / kBandDesc;
-        unsigned d0 = 0;
-        if (__lane_id() == 0) d0 = atomicAdd(ovf_cnt, nd);
-        d0 = (unsigned)__shfl((int)d0, 0);
-        const bool fits = d0 <= ovf_cap && nd <= ovf_cap - d0;
-        for (unsigned j = __lane_id(); j < nd && d0 + j < ovf_cap; j += 64)
-            ovf[d0 + j] = fits ? make_uint2(run_index + kBandWave + kBandDesc * j, min(kBandDesc, extra - kBandDesc * j))
-                               : make_uint2(0u, 0u);
-        if (fits) count = kBandWave;
-    }
-    for (unsigned i = __lane_id(); i < count; i += 64) {
-        const uint4 e = run[i];
-        mu[e.x] = mu_band(P, __uint_as_float(e.y), __uint_as_float(e.z));
-    }
-}
-
-// The interface entries beyond the first kBandWave of the runs of one mu launch: one
-// workgroup per descriptor of at most kBandDesc entries.  Also clears the descriptor
-// counter that the next launch posts to (cnt_next), so that no memset is needed.
-__global__ void __launch_bounds__(kBandDesc) k_band_overflow(const DevParams P, const uint4 *__restrict__ band,
-                                                             const uint2 *__restrict__ ovf,
-                                                             const unsigned *__restrict__ cnt,
-                                                             unsigned *__restrict__ cnt_next, float *__restrict__ mu,
-                                                             unsigned cap) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *cnt_next = 0u;
-    const unsigned n = min(*cnt, cap);
-    for (unsigned d = blockIdx.x; d < n; d += gridDim.x) {
-        const uint2 ds = ovf[d];
-        if (threadIdx.x < ds.y) {
-            const uint4 e = band[ds.x + threadIdx.x];
-            mu[e.x] = mu_band(P, __uint_as_float(e.y), __uint_as_float(e.z));
-        }
-    }
-}
-
-// one thread per node, stencil values from the caches
-// rho_solid (when given) is the buffer the next collide sums the density into;
-// its solid nodes receive this step's wall values.
-template <class TS>
-__global__ void __launch_bounds__(TPB) k_mu(const DevParams P, const TS *__restrict__ rho, TS *__restrict__ mu,
-                                            TS *__restrict__ rho_solid) {
-    const NodeIdx nd = node_from_grid(P);
-    if (!nd.ok) return;
-    const int I = (int)nd.I, pl = P.ny * P.nz;
-    if (is_solid(P, nd.z)) {
-        if (rho_solid) rho_solid[I] = rho[I];
-        return;
-    }
-    // 32-bit offsets of coordinate + s, s = -3..3 (periodic wrap folded in)
-    int ox[7], oy[7], oz[7];
-#pragma unroll
-    for (int s = 0; s < 7; ++s) {
-        ox[s] = (wrap_off(nd.x, s - 3, P.nx) - nd.x) * pl;
-        oy[s] = (wrap_off(nd.y, s - 3, P.ny) - nd.y) * P.nz;
-        oz[s] = wrap_off(nd.z, s - 3, P.nz) - nd.z;
-    }
-    mu[I] = mu_node<TS>(P, [&](int dx, int dy, int dz) { return rho[I + ox[dx + 3] + oy[dy + 3] + oz[dz + 3]]; });
-}
-
-
-// ---------------------------------------------------------------------------
 // Fused non-ideal force + MRT collision + exact-difference forcing + push
 // streaming with half-way bounce-back (NonidealForce + GlobalCollide,
 // FluidCuda.cu:311-347, 431-441).  u = j(f)/rho with rho the stored density.
@@ -558,197 +372,6 @@ __device__ __forceinline__ void ring_dest(int ly, int lz, int &dy, int &dz, int 
         if (lz == 0) { dz = -1; slot = slot_z1(ly - 1); }
         else { dz = 1; slot = slot_z0(ly - 1); }
     }
-}
-
-// Chemical potential as a march over the same tiles: rho of planes x-3..x+3 with an
-// in-plane halo of 3 sits in an LDS ring, so the 13 (or 19) stencil values of every
-// node come from LDS and each rho value is fetched from memory about once per tile.
-// Arithmetic of mu_node, as k_mu.
-// FIX (periodic FP32 lattices with the density summed by the collide kernel): rho
-// holds the previous collide's tile sums, which this kernel completes on the fly
-// with the terms k_density_fix adds (the ring entry and, on a chunk's first / last
-// plane, the partial-plane entry of the y-, z- and diagonal neighbour tile holding
-// the node, then the tile's own partial-plane entry: the same order, with +0 for
-// absent terms, so the same values) as each plane enters the ring; the completed
-// density of the workgroup's own tile and chunk is written to rho_out.  This
-// replaces the separate completion pass.
-template <class TS, bool FIX, int H>
-__global__ void __launch_bounds__(MT) k_mu_march(const DevParams P, const TS *__restrict__ rho, TS *__restrict__ mu,
-                                                  int ntz, int nty, TS *__restrict__ rho_solid, int xc,
-                                                  const TS *__restrict__ rbuf, const TS *__restrict__ cbuf,
-                                                  TS *__restrict__ rho_out, int nch, uint4 *__restrict__ band,
-                                                  uint2 *__restrict__ band_ovf, unsigned *__restrict__ band_cnt,
-                                                  unsigned band_cap) {
-    // ring of 2H+2 planes with an in-plane halo of H (2 for the 5-point Laplacian, 3 for
-    // the 7-point one): the stencil reads 2H+1 of them, and the extra slot lets the
-    // plane entering the ring be stored while slower waves still read the plane that
-    // left it, so one barrier per plane suffices
-    constexpr int R = 2 * H + 2, LZ = MTZ + 2 * H, LP = (MTY + 2 * H) * LZ;
-    __shared__ TS s_rho[R][LP];
-    // FP32: this wave's run of interface nodes and their count
-    const unsigned run_index = (unsigned)(((size_t)blockIdx.x * (MT / 64) + threadIdx.x / 64) * 64 * xc);
-    uint4 *band_run = band ? band + run_index : nullptr;
-    unsigned band_count = 0;
-    int t = blockIdx.x;
-    if ((gridDim.x & 7) == 0) t = (t & 7) * (gridDim.x >> 3) + (t >> 3);
-    const int tzi = t % ntz;
-    t /= ntz;
-    const int tyi = t % nty;
-    const int ch = t / nty;
-    const int y0 = tyi * MTY, z0 = tzi * MTZ;
-    const int xa = ch * xc, xb = min(xa + xc, P.nx);
-    const int ty = threadIdx.x / MTZ, tz = threadIdx.x % MTZ;
-    const int y = y0 + ty, z = z0 + tz;
-    const bool inr = (y < P.ny) && (z < P.nz);
-    const bool active = inr && !is_solid(P, z);
-    constexpr int HE = (LP + MT - 1) / MT;
-    int hoff[HE];
-    // FIX: in-plane part of the ring index of the (up to three) neighbouring tiles
-    // holding each halo node (y-, z-, diagonal neighbour), -1 where absent
-    int ro[FIX ? HE : 1][3];
-    // and of their partial-plane entries (slot 3: the node's own tile), without the
-    // chunk and side, which are uniform per plane
-    int co[FIX ? HE : 1][4];
-    const long long plane_ring = (long long)nty * ntz * ARING;
-#pragma unroll
-    for (int h = 0; h < HE; ++h) {
-        const int e = threadIdx.x + h * MT;
-        const int ly = e / LZ, lz = e - ly * LZ;
-        const int hy = e < LP ? wrapc(y0 - H + ly, P.ny) : 0;
-        const int hz = e < LP ? wrapc(z0 - H + lz, P.nz) : 0;
-        hoff[h] = hy * P.nz + hz;
-        if constexpr (FIX) {
-            const int gyi = hy / MTY, gzi = hz / MTZ, gy = hy % MTY, gz = hz % MTZ;
-            const bool ey0 = gy == 0, ey1 = gy == MTY - 1, ez0 = gz == 0, ez1 = gz == MTZ - 1;
-            const int own_ring = (gyi * ntz + gzi) * ARING;
-            auto set = [&](int i, bool on, int dy, int dz, int ly2, int lz2, int slot) {
-                if (!on) return;
-                const int yy = (gyi + dy + nty) % nty, zz = (gzi + dz + ntz) % ntz;
-                ro[h][i] = own_ring + slot;
-                co[h][i] = (yy * ntz + zz) * 2 * AP + ly2 * AZ + lz2;
-            };
-            ro[h][0] = ro[h][1] = ro[h][2] = -1;
-            co[h][0] = co[h][1] = co[h][2] = 0;
-            set(0, ey0, -1, 0, AY - 1, gz + 1, slot_y0(gz));
-            set(0, ey1, 1, 0, 0, gz + 1, slot_y1(gz));
-            set(1, ez0, 0, -1, gy + 1, AZ - 1, slot_z0(gy));
-            set(1, ez1, 0, 1, gy + 1, 0, slot_z1(gy));
-            set(2, ey0 && ez0, -1, -1, AY - 1, AZ - 1, slot_c(-1, -1));
-            set(2, ey0 && ez1, -1, 1, AY - 1, 0, slot_c(-1, 1));
-            set(2, ey1 && ez0, 1, -1, 0, AZ - 1, slot_c(1, -1));
-            set(2, ey1 && ez1, 1, 1, 0, 0, slot_c(1, 1));
-            co[h][3] = (gyi * ntz + gzi) * 2 * AP + (gy + 1) * AZ + gz + 1;
-        }
-    }
-    // planes xg of the march, xa - H .. xb + H + 1, wrapped into [0, nx) without a
-    // division once the lattice is at least 8 planes long
-    const bool long_x = P.nx >= 8;
-    auto wrap_x = [&](int xg) { return long_x ? (xg < 0 ? xg + P.nx : (xg >= P.nx ? xg - P.nx : xg)) : wrapc(xg, P.nx); };
-    // two planes in flight: the halo of planes x+H+1 and x+H+2 while plane x
-    // computes (register sets A and B alternate; the loop is unrolled by two so
-    // that they keep fixed registers)
-    TS hA[HE], hB[HE];
-    TS fA[FIX ? HE : 1][3], fB[FIX ? HE : 1][3];
-    auto fetch_plane = [&](int xg, TS *hr, TS (*fv)[3]) {   // wraps past the chunk (loads unused then)
-        xg = wrap_x(xg);
-        const TS *rp = rho + (long long)xg * P.ny * P.nz;
-        const TS *fp = FIX ? rbuf + (long long)xg * plane_ring : nullptr;   // ring entries of plane xg
-#pragma unroll
-        for (int h = 0; h < HE; ++h)
-            if ((h + 1) * MT <= LP || threadIdx.x + h * MT < LP) {
-                hr[h] = rp[hoff[h]];
-                if constexpr (FIX) {
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) fv[h][i] = ro[h][i] >= 0 ? fp[ro[h][i]] : TS(0);
-                }
-            }
-    };
-    // the planes enter the ring in order xa - H, xa - H + 1, ...: the wrapped plane,
-    // its position in its chunk and its chunk advance by one per stored plane
-    int st_xw = wrap_x(xa - H), st_k = 0, st_ch = 0;
-    if constexpr (FIX) {
-        st_k = st_xw % xc;
-        st_ch = st_xw / xc;
-    }
-    auto store_plane = [&](int slot, const TS *hr, TS (*fv)[3]) {
-        const int k = st_k;
-        const bool chunk_end = k == 0 || k == xc - 1;   // partial-plane terms too (uniform)
-#pragma unroll
-        for (int h = 0; h < HE; ++h)
-            if ((h + 1) * MT <= LP || threadIdx.x + h * MT < LP) {
-                TS v = hr[h];
-                if constexpr (FIX) {
-                    // k_density_fix's order: ring and partial-plane entry of each
-                    // neighbour, then the own partial-plane entry (+0 off the chunk ends)
-                    TS a = TS(0);
-                    if (chunk_end) {
-                        const int cs = k == 0 ? (st_ch == 0 ? nch - 1 : st_ch - 1) : (st_ch == nch - 1 ? 0 : st_ch + 1);
-                        const long long ub = ((long long)cs * nty * ntz * 2 + (k == 0 ? 1 : 0)) * AP;
-#pragma unroll
-                        for (int i = 0; i < 3; ++i) {
-                            const TS c = cbuf[ub + co[h][i]];
-                            a += fv[h][i];
-                            a += ro[h][i] >= 0 ? c : TS(0);
-                        }
-                        a += cbuf[ub + co[h][3]];
-                    } else {
-                        a += fv[h][0];
-                        a += fv[h][1];
-                        a += fv[h][2];
-                    }
-                    v = v + a;
-                }
-                s_rho[slot][threadIdx.x + h * MT] = v;
-            }
-        // next plane
-        st_xw = st_xw + 1 == P.nx ? 0 : st_xw + 1;
-        if constexpr (FIX) {
-            if (++st_k == xc || st_xw == 0) {
-                st_k = 0;
-                st_ch = st_xw == 0 ? 0 : st_ch + 1;
-            }
-        }
-    };
-    for (int k = -H; k < H; ++k) { fetch_plane(xa + k, hA, fA); store_plane(k + H, hA, fA); }
-    fetch_plane(xa + H, hA, fA);
-    fetch_plane(xa + H + 1, hB, fB);
-    const int base = (ty + H) * LZ + tz + H;
-    const int ym = y < P.ny ? y : 0, zm = z < P.nz ? z : 0;
-    // ring slot of plane x - H is rs0 (plane p sits in slot (p - xa + H) % R)
-    int rs0 = 0;
-    auto plane_step = [&](int x, TS *hr, TS (*fv)[3]) {
-        int slot[R];
-#pragma unroll
-        for (int dd = 0; dd < R; ++dd) slot[dd] = rs0 + dd >= R ? rs0 + dd - R : rs0 + dd;
-        store_plane(slot[2 * H], hr, fv);                    // plane x+H
-        __syncthreads();
-        fetch_plane(x + 2 + H, hr, fv);                      // plane x+H+2
-        const long long I = ((long long)x * P.ny + ym) * P.nz + zm;
-        float kal = 0.0f;
-        if (active) {
-            mu[I] = mu_node<TS, false>(P, [&](int dx, int dy, int dz) { return s_rho[slot[dx + H]][base + dy * LZ + dz]; },
-                                       &kal);
-        } else if (rho_solid && inr) {
-            rho_solid[I] = s_rho[slot[H]][base];
-        }
-        if constexpr (sizeof(TS) == 4)
-            if (band) {
-                const float dcen = s_rho[slot[H]][base];
-                band_append(active && in_band(P, dcen), (unsigned)I, dcen, kal, band_run, band_count);
-            }
-        // rho_out (if given) receives the density of the node: with FIX the completed
-        // one, without a copy of rho (the adjoint's tape)
-        if (rho_out && inr) rho_out[I] = s_rho[slot[H]][base];
-        rs0 = rs0 + 1 == R ? 0 : rs0 + 1;
-    };
-    int x = xa;
-    for (; x + 1 < xb; x += 2) {
-        plane_step(x, hA, fA);
-        plane_step(x + 1, hB, fB);
-    }
-    if (x < xb) plane_step(x, hA, fA);
-    if constexpr (sizeof(TS) == 4)
-        if (band) band_finish(P, band_run, band_count, (float *)mu, run_index, band_ovf, band_cnt, band_cap);
 }
 
 // With RS the kernel also sums the next step's density: every post-collision
@@ -1549,17 +1172,6 @@ hipError_t launch_wall(cpmp_ctx *c) {
     });
 }
 
-// CPMP_COLLIDE=v1 / CPMP_MU=v1 select the one-thread-per-node kernels (stencils
-// from cache) instead of the LDS marches
-static int variant(const char *var) {
-    const char *e = std::getenv(var);
-    return (e && std::strcmp(e, "v1") == 0) ? 1 : 2;
-}
-static int mu_variant() {
-    static const int v = variant("CPMP_MU");
-    return v;
-}
-
 // FP32 storage forms with the march collide sum the density inside the collide
 // kernel when the tiles cover the lattice exactly (a context created with
 // CPMP_FUSE=0 in the environment keeps the separate density pass)
@@ -1619,62 +1231,19 @@ template <class TS> static const TS *ref_buffer(const cpmp_ctx *c) {
     return c->form == CPMP_FORM_FP16 ? (const TS *)c->rho_next : nullptr;
 }
 
-// after a mu march with interface runs: the entries its waves posted as overflow, then
-// the other descriptor counter for the next launch
-static hipError_t launch_band_overflow(cpmp_ctx *c) {
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const int par = c->band_par;
-    // a grid of 2048 workgroups (8 per CU) strides over the descriptors: ~2100 at 256^3
-    hipLaunchKernelGGL(k_band_overflow, dim3(2048), dim3(kBandDesc), 0, c->stream, c->dp, (const uint4 *)c->band,
-                       (const uint2 *)c->band_ovf, (const unsigned *)(c->band_cnt + par), c->band_cnt + (par ^ 1),
-                       (float *)c->mu, c->band_cap);
-    c->band_par = par ^ 1;
-    return hipGetLastError();
-}
-
-hipError_t launch_mu(cpmp_ctx *c, void *rho_copy) {
-    return dispatch(c->form, [&](auto fm) {
-        using TS = typename decltype(fm)::TS;
-        TS *solid = (TS *)c->rho_next;   // double-buffered density: solid values follow the step
-        if (mu_variant() == 1) {
-            if (rho_copy) {
-                const hipError_t e = hipMemcpyAsync(rho_copy, c->rho, (size_t)c->N * sizeof(TS), hipMemcpyDeviceToDevice,
-                                                    c->stream);
-                if (e != hipSuccess) return e;
-            }
-            hipLaunchKernelGGL(k_mu<TS>, node_grid(c->dp), dim3(TPB), 0, c->stream, c->dp, (const TS *)c->rho,
-                               (TS *)c->mu, solid);
-        } else {
-            const int xc = c->dp.xc;   // shorter chunks measured slower (0.077 vs 0.071 ms at 256^3)
-            const int ntz = (c->p.nz + MTZ - 1) / MTZ, nty = (c->p.ny + MTY - 1) / MTY, nch = (c->p.nx + xc - 1) / xc;
-            auto go = [&](auto h_t) {
-                hipLaunchKernelGGL((k_mu_march<TS, false, decltype(h_t)::value>), dim3((unsigned)(ntz * nty * nch)),
-                                   dim3(MT), 0, c->stream, c->dp, (const TS *)c->rho, (TS *)c->mu, ntz, nty, solid, xc,
-                                   (const TS *)nullptr, (const TS *)nullptr, (TS *)rho_copy, nch, c->band, c->band_ovf,
-                                   c->band_cnt ? c->band_cnt + c->band_par : nullptr, c->band_cap);
-            };
-            if (c->dp.lap_points == 7) go(std::integral_constant<int, 3>{});
-            else go(std::integral_constant<int, 2>{});
-            if (c->band) return launch_band_overflow(c);
-        }
-        return hipGetLastError();
-    });
-}
-
 bool moment_path(const cpmp_params &p, const DevParams &d, bool fuse_off, bool covered) {
     const char *e = std::getenv("CPMP_COLLIDE");
     if (!d.unit_rates || p.form == CPMP_FORM_FP16 || (e && std::strcmp(e, "v1") == 0) || (fuse_off && covered)) return false;
     return d.N >= 100000 || (e && std::strcmp(e, "march") == 0) || std::getenv("CPMP_XC");
 }
 
-hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool keep_sums, bool first, bool last) {
+hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool last) {
     if (c->moments) {
-        const hipError_t e = launch_moment_step(c, first, last, want_mv, uout_v);
-        c->cur ^= 1;
+        const hipError_t e = launch_moment_step(c, last, want_mv, uout_v);
         std::swap(c->rho, c->rho_next);
         return e;
     }
+    c->mom_at = 0;
     const bool rs = density_fused(c);
     const hipError_t e = dispatch(c->form, [&](auto fm) {
         using TF = typename decltype(fm)::TF;
@@ -1753,9 +1322,8 @@ hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool keep_sum
         return hipGetLastError();
     });
     c->cur ^= 1;
-    // the summed density is now current (keep_sums: it stays in rho_next for the
-    // next mu kernel to complete)
-    if (rs && !keep_sums) std::swap(c->rho, c->rho_next);
+    // the summed density is now current
+    if (rs) std::swap(c->rho, c->rho_next);
     return e;
 }
 
@@ -1785,50 +1353,14 @@ hipError_t launch_macro(cpmp_ctx *c) {
     return e;
 }
 
-// Periodic FP32 lattices with the density summed by the collide kernel: within a
-// run of steps the completion of each step's density (k_density_fix) is folded
-// into the next step's mu kernel (k_mu_march<float, true>); the last step of the
-// run completes its density as usual, so the state between runs is the same.
-// CPMP_DEFER=0 turns this off.
-static bool fix_deferrable(const cpmp_ctx *c) {
-    const char *env = std::getenv("CPMP_DEFER");
-    const bool off = env && std::strcmp(env, "0") == 0;
-    return !off && density_fused(c) && c->form == CPMP_FORM_FP32 && c->dp.lo == 0 && c->dp.hi == 0 &&
-           mu_variant() != 1 && c->dp.xc >= 2;
-}
-
-// the previous collide's tile sums (rho_next) completed into rho, and mu from them
-static hipError_t launch_mu_fix(cpmp_ctx *c) {
-    const int xc = c->dp.xc, ntz = c->p.nz / MTZ, nty = c->p.ny / MTY, nch = c->p.nx / xc;
-    auto go = [&](auto h_t) {
-        hipLaunchKernelGGL((k_mu_march<float, true, decltype(h_t)::value>), dim3((unsigned)(ntz * nty * nch)), dim3(MT), 0,
-                           c->stream, c->dp, (const float *)c->rho_next, (float *)c->mu, ntz, nty, (float *)nullptr, xc,
-                           (const float *)c->rbuf, (const float *)c->cbuf, (float *)c->rho, nch, c->band, c->band_ovf,
-                           c->band_cnt ? c->band_cnt + c->band_par : nullptr, c->band_cap);
-    };
-    if (c->dp.lap_points == 7) go(std::integral_constant<int, 3>{});
-    else go(std::integral_constant<int, 2>{});
-    if (c->band) return launch_band_overflow(c);
-    return hipGetLastError();
-}
-
 hipError_t launch_steps(cpmp_ctx *c, int nsteps, bool want_mv) {
-    const bool defer = fix_deferrable(c);
     hipError_t e;
     for (int n = 0; n < nsteps; ++n) {
         const bool last = n == nsteps - 1;
-        if (defer && n > 0) {
-            if ((e = launch_mu_fix(c)) != hipSuccess) return e;
-        } else {
-            if ((e = launch_wall(c)) != hipSuccess) return e;
-            if ((e = launch_mu(c)) != hipSuccess) return e;
-        }
-        if (defer && !last) {
-            if ((e = launch_collide(c, false, nullptr, true)) != hipSuccess) return e;
-        } else {
-            if ((e = launch_collide(c, last && want_mv, nullptr, false, n == 0, last)) != hipSuccess) return e;
-            if ((e = launch_macro(c)) != hipSuccess) return e;
-        }
+        if ((e = launch_wall(c)) != hipSuccess) return e;
+        if ((e = launch_mu(c)) != hipSuccess) return e;
+        if ((e = launch_collide(c, last && want_mv, nullptr, last)) != hipSuccess) return e;
+        if ((e = launch_macro(c)) != hipSuccess) return e;
     }
     return hipSuccess;
 }

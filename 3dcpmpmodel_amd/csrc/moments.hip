@@ -4,11 +4,12 @@
 // With rate 1 on rows 0, 1, 3, 5, 7, 10, 12 and 16..18 the collision reads of the
 // pulled populations only the density, the momentum (rows 3, 5, 7) and the nine rows
 // 2, 4, 6, 8, 9, 11, 13, 14, 15.  Within a run of steps these are what a step hands to
-// the next: the density array and 12 moments per node.  The first step of a run reads
-// the populations, the last one writes them, so that between calls the state is the
-// populations as everywhere else in the library.  Every variant forms a node's moments
-// from its 19 pulled values with the same operations, and floating contraction is
-// limited to single expressions (below), so a run rounds the same however it is split.
+// the next: the density array and 12 moments per node.  The last step of a call also
+// writes the populations, the state that the rest of the library reads and writes; a step
+// after any of these has written them starts from the populations.  Every variant forms a
+// node's moments from its 19 pulled values with the same operations, and floating
+// contraction is limited to single expressions (below), so a run rounds the same however
+// it is split.
 #pragma clang fp contract(on)
 
 #include "internal.h"
@@ -142,15 +143,14 @@ enum { kPlain, kQp, kGuo };   // force term: exact difference, with Qp, Guo (Qp 
 // collides every node of its tile and of the ring of neighbours around it, posts the 16
 // populations that leave their column in an LDS mailbox, and each own node collects what
 // arrives: after the plane behind it has collided, a node holds its 19 pulled values and
-// writes their moments (OUT_P: the post-collision populations are written instead, and
-// of the arrivals only the density).  Nothing is exchanged between workgroups within a
+// writes their moments (OUT_P: its post-collision populations too).  Nothing is exchanged between workgroups within a
 // step, so any lattice size works and no density completion follows; the price is the
 // ring: 340 collisions for 256 nodes, and two more planes per chunk.
 template <class TF, class TS, class TC, class TL, bool IN_P, bool OUT_P, bool DIAG, bool NW, int FC>
-__global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 && !IN_P ? 4 : 2) k_moment_step(const DevParams P, const StepArgs<TF, TS, TC> A) {
+__global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 ? 4 : 2) k_moment_step(const DevParams P, const StepArgs<TF, TS, TC> A) {
     __shared__ Pair<TC> s_rm[7][TL::EP];       // planes x-3 .. x+3
     __shared__ TC s_mail[Q - 3][TL::NN];       // populations 3..18 of plane x
-    __shared__ TC s_edge[OUT_P ? 1 : 2 * kMom * TL::TY];   // edge columns of a finished plane
+    __shared__ TC s_edge[2 * kMom * TL::TY];   // edge columns of a finished plane
     int t = blockIdx.x;
     {
         // workgroup b runs on XCD b % 8: each XCD takes a contiguous range of tiles (z
@@ -252,7 +252,7 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 && !IN_P ? 4 : 2) k_mo
         TC r7[7][TL::HE], m7[7][TL::HE];
 #pragma unroll
         for (int k = 0; k < 7; ++k) fetch_plane(xa - 4 + k, r7[k], m7[k]);
-        fetch_state(xa - 1);
+        if constexpr (!IN_P) fetch_state(xa - 1);
 #pragma unroll
         for (int k = 0; k < 7; ++k) store_plane(k, r7[k], m7[k]);
     }
@@ -261,12 +261,10 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 && !IN_P ? 4 : 2) k_mo
     const int one = z0 == zlast ? kMom * TL::TY : TL::NT;
     // a finished plane's edge columns, from LDS to memory
     auto flush_edges = [&](int xp) {
-        if constexpr (!OUT_P) {
-            static_assert(2 * kMom * TL::TY <= TL::NT, "one value per thread");
-            TC *b = A.eout + ((size_t)xp * tiles + tile) * (2 * kMom * TL::TY);
-            // a tile of one column keeps it as its first
-            if (tid < 2 * kMom * TL::TY) *lane_at(b, (unsigned)tid) = s_edge[tid - (tid >= one ? kMom * TL::TY : 0)];
-        }
+        static_assert(2 * kMom * TL::TY <= TL::NT, "one value per thread");
+        TC *b = A.eout + ((size_t)xp * tiles + tile) * (2 * kMom * TL::TY);
+        // a tile of one column keeps it as its first
+        if (tid < 2 * kMom * TL::TY) *lane_at(b, (unsigned)tid) = s_edge[tid - (tid >= one ? kMom * TL::TY : 0)];
     };
     const int base = (TL::flat ? 0 : (ly + 3) * TL::ES) + lz + 3;
 
@@ -283,14 +281,17 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 && !IN_P ? 4 : 2) k_mo
     __syncthreads();
 
     for (int x = xa - 1; x <= xb; ++x) {
+        // moments are loaded a plane ahead (past the chunk wrapped, and not used); the
+        // populations of a run's first step at the start of their own plane, behind the
+        // stencils, which keeps 19 registers free and a second workgroup on the CU
         TC m[Q];
         if constexpr (IN_P) {
-            moments(next, m);
+            fetch_state(x);
         } else {
 #pragma unroll
             for (int k = 0; k < kMom; ++k) m[mom_row(k)] = next[k];
+            fetch_state(x + 1);
         }
-        fetch_state(x + 1);       // loads past the chunk are issued (wrapped) and not used
         if (x > xa + 1) flush_edges(x - 2);
         TC out[Q];
         if (fluid) {
@@ -300,6 +301,7 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 && !IN_P ? 4 : 2) k_mo
             const RingStencil<TC, TL> st{s_rm, slot, base};
             TC gr[3], gm[3], u[3];
             st.grad(gr, gm);
+            if constexpr (IN_P) moments(next, m);
             const TC r = st.at(0, 0, 0).r, third = TC(1.0 / 3.0);
             const TC Fx = gr[0] * third - gm[0] * r, Fy = gr[1] * third - gm[1] * r, Fz = gr[2] * third - gm[2] * r;
             if (FC != kPlain && P.qp_on) {
@@ -336,7 +338,7 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 && !IN_P ? 4 : 2) k_mo
             if (own && x >= xa && x < xb) {
                 const unsigned b = (unsigned)x * (unsigned)pl + psite;
 #pragma unroll
-                for (int q = 0; q < Q; ++q) A.fout[(unsigned)q * (unsigned)P.N + b] = (TF)out[q];
+                for (int q = 0; q < Q; ++q) __builtin_nontemporal_store((TF)out[q], &A.fout[(unsigned)q * (unsigned)P.N + b]);
             }
         }
         __syncthreads();                       // mailbox of plane x posted, plane x - 3 no longer read
@@ -361,14 +363,12 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 && !IN_P ? 4 : 2) k_mo
                 TC n[Q];
                 moments(fa, n);
                 const int xp = x - 1;
-                if constexpr (!OUT_P) {
-                    TC *b = A.mout + (size_t)xp * kMom * pl;
+                TC *b = A.mout + (size_t)xp * kMom * pl;
 #pragma unroll
-                    for (int k = 0; k < kMom; ++k) {
-                        const TC v = fluid ? n[mom_row(k)] : TC(0);
-                        __builtin_nontemporal_store(v, lane_at(b + (size_t)k * pl, site));
-                        if (edge) s_edge[k * TL::TY + eslot] = v;
-                    }
+                for (int k = 0; k < kMom; ++k) {
+                    const TC v = fluid ? n[mom_row(k)] : TC(0);
+                    __builtin_nontemporal_store(v, lane_at(b + (size_t)k * pl, site));
+                    if (edge) s_edge[k * TL::TY + eslot] = v;
                 }
                 if (fluid) *lane_at(A.rho_out + (size_t)xp * pl, node) = (TS)n[0];
             }
@@ -406,10 +406,15 @@ template <class TF, class TS, class TC>
 hipError_t launch_form(cpmp_ctx *c, bool in_p, bool out_p, double *mv, TS *uout) {
     const DevParams &P = c->dp;
     StepArgs<TF, TS, TC> a;
+    // moments alternate between c->mom and the population set that is not current; the
+    // populations of the last step replace the current ones, which nothing reads any
+    // more unless this step starts from them
+    const void *in = c->mom_at == 1 ? c->mom : c->f[c->cur ^ 1];
+    void *out = c->mom_at == 1 ? c->f[c->cur ^ 1] : c->mom;
     a.fin = (const TF *)c->f[c->cur];
-    a.min = (const TC *)c->f[c->cur];
-    a.fout = (TF *)c->f[c->cur ^ 1];
-    a.mout = (TC *)c->f[c->cur ^ 1];
+    a.fout = (TF *)c->f[in_p ? c->cur ^ 1 : c->cur];
+    a.min = (const TC *)in;
+    a.mout = (TC *)out;
     a.ein = a.min + (size_t)kMom * c->N;   // the edge columns follow the moments
     a.eout = a.mout + (size_t)kMom * c->N;
     a.rho = (const TS *)c->rho;
@@ -476,14 +481,25 @@ int moment_chunk(int nx, int ny, int nz, int form) {
     return best;
 }
 
-hipError_t launch_moment_step(cpmp_ctx *c, bool in_pops, bool out_pops, bool want_mv, void *uout) {
+// values of a moment set: 12 per node and the edge columns of every tile
+size_t moment_bytes(int nx, int ny, int nz, int form) {
+    const int ty = ny == 1 ? TileRow::TY : TileBox::TY, tz = ny == 1 ? TileRow::TZ : TileBox::TZ;
+    const size_t tiles = (size_t)((ny + ty - 1) / ty) * ((nz + tz - 1) / tz);
+    return (size_t)nx * kMom * ((size_t)ny * nz + tiles * 2 * ty) * (form == CPMP_FORM_FP64 ? 8 : 4);
+}
+
+hipError_t launch_moment_step(cpmp_ctx *c, bool out_pops, bool want_mv, void *uout) {
     double *mv = want_mv ? c->mv : nullptr;
+    const bool in_pops = c->mom_at == 0;
+    hipError_t e = hipErrorInvalidValue;
     switch (c->form) {
-    case CPMP_FORM_FP64: return launch_form<double, double, double>(c, in_pops, out_pops, mv, (double *)uout);
-    case CPMP_FORM_FP32: return launch_form<float, float, float>(c, in_pops, out_pops, mv, (float *)uout);
-    case CPMP_FORM_FP32A: return launch_form<double, double, float>(c, in_pops, out_pops, mv, (double *)uout);
+    case CPMP_FORM_FP64: e = launch_form<double, double, double>(c, in_pops, out_pops, mv, (double *)uout); break;
+    case CPMP_FORM_FP32: e = launch_form<float, float, float>(c, in_pops, out_pops, mv, (float *)uout); break;
+    case CPMP_FORM_FP32A: e = launch_form<double, double, float>(c, in_pops, out_pops, mv, (double *)uout); break;
     }
-    return hipErrorInvalidValue;
+    if (in_pops && out_pops) c->cur ^= 1;
+    c->mom_at = c->mom_at == 1 ? 2 : 1;
+    return e;
 }
 
 }  // namespace cpmp

@@ -22,7 +22,7 @@ CASES = [
     ((7, 11, 31), 7, 0, {}),                    # below one tile; nx below 8 (general wrap)
     ((1, 24, 64), 1, 0, {}),
     ((5, 25, 65), 2, 0, dict(lap_points=7)),
-    ((10, 2, 40), 10, 3, dict(wall_scheme=0)),
+    ((10, 3, 40), 10, 3, dict(wall_scheme=0)),
     ((16, 14, 20), 64, 3, dict(wall_scheme=2)),
     ((12, 13, 34), 5, 3, dict(K1=0.003, K2=-0.003)),
     ((12, 23, 24), 5, 3, dict(forcing=1)),
