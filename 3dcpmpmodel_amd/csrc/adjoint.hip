@@ -634,6 +634,7 @@ int make_plan(cpmp_ctx *c, const cpmp_adj_desc *d, AdjPlan &q) {
     if (need_free) {
         const hipError_t e = hipMemGetInfo(&fr, &tot);
         if (e != hipSuccess) return set_error(CPMP_EHIP, "hipMemGetInfo: %s", hipGetErrorString(e));
+        fr += c->adj_ws_bytes;   // the kept workspace is reused or returned first
     }
     long long budget = d->tape_budget_bytes < 0 ? (long long)(fr / 2) : d->tape_budget_bytes;
     q.ntaped = (int)std::min<long long>(budget / (long long)q.per_tape, d->nsteps);
@@ -753,6 +754,7 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
     const size_t sb = c->scal_bytes;
     char *ckpt = nullptr, *subck = nullptr, *fin = nullptr, *tape = nullptr, *tape2 = nullptr;
     double *buf = nullptr, *tgt = nullptr;
+    bool kept = false;
     // overlapped schedule: the recompute runs on the context's state on stream s2
     hipStream_t s2 = nullptr;
     hipEvent_t ev_first = nullptr, ev_tape[2] = {nullptr, nullptr}, ev_rev[2] = {nullptr, nullptr};
@@ -760,12 +762,32 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
     double *rb, *rbn, *rbl, *Pf, *Wf, *mub, *part, *kpart, *gl, *gh, *acc;
     double acc_h[2] = {0, 0};
     {
-        AHIP(hipMalloc((void **)&ckpt, (size_t)std::max(q.nseg, 1) * q.per_ck));
-        if (q.nsubck > 0) AHIP(hipMalloc((void **)&subck, (size_t)q.nsubck * q.per_ck));
-        AHIP(hipMalloc((void **)&fin, q.per_ck));
-        AHIP(hipMalloc((void **)&tape, (size_t)q.tape_len * q.per_tape));
+        // the parts of the workspace, in one block where it is kept
+        struct { char **p; size_t n; } part_of[] = {
+            {&ckpt, (size_t)std::max(q.nseg, 1) * q.per_ck}, {&subck, (size_t)q.nsubck * q.per_ck}, {&fin, q.per_ck},
+            {&tape, (size_t)q.tape_len * q.per_tape}, {&tape2, q.pipe ? (size_t)q.tape_len * q.per_tape : 0},
+            {(char **)&buf, q.nbuf * sizeof(double)}, {(char **)&tgt, (size_t)N * sizeof(double)}};
+        auto padded = [](size_t n) { return (n + 255) / 256 * 256; };
+        size_t need = 0;
+        for (auto &w : part_of) need += padded(w.n);
+        kept = need <= kAdjKeep;
+        if (c->adj_ws && (!kept || c->adj_ws_bytes < need)) {
+            (void)hipFree(c->adj_ws);
+            c->adj_ws = nullptr;
+            c->adj_ws_bytes = 0;
+        }
+        if (kept && !c->adj_ws) {
+            AHIP(hipMalloc((void **)&c->adj_ws, need));
+            c->adj_ws_bytes = need;
+        }
+        size_t at = 0;
+        for (auto &w : part_of) {
+            if (w.n == 0) continue;
+            if (kept) *w.p = c->adj_ws + at;
+            else AHIP(hipMalloc((void **)w.p, w.n));
+            at += padded(w.n);
+        }
         if (q.pipe) {
-            AHIP(hipMalloc((void **)&tape2, (size_t)q.tape_len * q.per_tape));
             AHIP(hipStreamCreateWithFlags(&s2, hipStreamNonBlocking));
             AHIP(hipEventCreateWithFlags(&ev_first, hipEventDisableTiming));
             for (int i = 0; i < 2; ++i) {
@@ -773,8 +795,6 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
                 AHIP(hipEventCreateWithFlags(&ev_rev[i], hipEventDisableTiming));
             }
         }
-        AHIP(hipMalloc((void **)&buf, q.nbuf * sizeof(double)));
-        AHIP(hipMalloc((void **)&tgt, N * sizeof(double)));
         {
             double *p = buf;
             // folded population cotangents: two sets of 19 N values of hb bytes
@@ -961,12 +981,8 @@ done:
     }
     for (hipEvent_t ev : {ev_first, ev_tape[0], ev_tape[1], ev_rev[0], ev_rev[1]})
         if (ev) (void)hipEventDestroy(ev);
-    if (tape2) (void)hipFree(tape2);
-    if (ckpt) (void)hipFree(ckpt);
-    if (subck) (void)hipFree(subck);
-    if (fin) (void)hipFree(fin);
-    if (tape) (void)hipFree(tape);
-    if (buf) (void)hipFree(buf);
-    if (tgt) (void)hipFree(tgt);
+    if (!kept)
+        for (void *w : {(void *)ckpt, (void *)subck, (void *)fin, (void *)tape, (void *)tape2, (void *)buf, (void *)tgt})
+            if (w) (void)hipFree(w);
     return rc;
 }

@@ -325,7 +325,7 @@ int cpmp_destroy(cpmp_ctx *c) {
     if (!c) return CPMP_OK;
     if (c->stream) { hipSetDevice(c->p.device); hipStreamSynchronize(c->stream); }
     for (void *ptr : {c->f[0], c->f[1], c->rho, c->rho_next, c->rbuf, c->cbuf, c->mom, c->mu, (void *)c->mv, (void *)c->mu_w,
-                      (void *)c->red, (void *)c->staging})
+                      (void *)c->red, (void *)c->staging, (void *)c->adj_ws})
         if (ptr) hipFree(ptr);
     if (c->timers) {
         for (auto &e : c->timers->ev) if (e) hipEventDestroy(e);

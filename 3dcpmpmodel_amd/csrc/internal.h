@@ -68,6 +68,9 @@ struct cpmp_ctx {
     void *mom = nullptr;
     int mom_at = 0;
     size_t fuse_bytes = 0;
+    // workspace of the adjoint, kept for the next call up to kAdjKeep bytes
+    char *adj_ws = nullptr;
+    size_t adj_ws_bytes = 0;
     double *mv = nullptr;       // 3*N, MV of the last step
     double *mu_w = nullptr;     // 2*NXY: bottom then top
     double *red = nullptr;      // reduction partials
@@ -112,6 +115,10 @@ size_t moment_bytes(int nx, int ny, int nz, int form);
 // the populations, to moments and (out_pops) populations; rho_next receives the new
 // density of the fluid nodes
 hipError_t launch_moment_step(cpmp_ctx *c, bool out_pops, bool want_mv, void *uout);
+// Adjoint workspaces up to this size stay with the context: allocating and freeing them
+// took 3 to 50 ms a call, more than the sweep of a small lattice (128x128x64 FP32, 40 taped
+// steps: 54 ms a call, 13.7 ms of it work); larger ones are returned after the call.
+constexpr size_t kAdjKeep = (size_t)8 << 30;
 constexpr int kTileY = 8, kTileZ = 32;   // in-plane tile of the march kernels and of tiled population storage
 constexpr int kWallTile = 16;             // columns per edge of the wall-fill tiles (16 x 16 workgroups)
 // copy one population set between the device layout and the reference node order
