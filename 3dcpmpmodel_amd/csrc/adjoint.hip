@@ -470,7 +470,7 @@ __global__ void __launch_bounds__(TPB) k_adj_wall_pass(const DevParams P, double
     }
 }
 
-// The transposed fill in one launch for walls of at most R (<= 3) layers, over
+// The transposed fill in one launch for walls of at most R (<= 4) layers, over
 // 16 x 16 tiles of columns (blockIdx.z: 0 bottom wall, 1 top wall).  Layered
 // scheme: the first fluid layer gains A(rb(1) + A(rb(2) + A rb(3))), rb(d) the
 // cotangent of the solid layer at depth d and A the symmetric diagonal average;
@@ -869,6 +869,8 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
                     hipLaunchKernelGGL(k_adj_wall_tile<2>, gwt, bwt, 0, s, P, rbn, (const double *)mub, gl, gh);
                 else if (passes == 3)
                     hipLaunchKernelGGL(k_adj_wall_tile<3>, gwt, bwt, 0, s, P, rbn, (const double *)mub, gl, gh);
+                else if (passes == 4)
+                    hipLaunchKernelGGL(k_adj_wall_tile<4>, gwt, bwt, 0, s, P, rbn, (const double *)mub, gl, gh);
                 else
                     for (int pass = passes - 1; pass >= 0; --pass)
                         hipLaunchKernelGGL(k_adj_wall_pass, dim3(nbc), dim3(TPB), 0, s, P, rbn, pass,

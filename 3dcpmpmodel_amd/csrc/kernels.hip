@@ -132,8 +132,8 @@ __global__ void __launch_bounds__(TPB) k_wall(const DevParams P, TS *__restrict_
     }
 }
 
-// The same fill in one launch for walls of at most R (<= 3) layers.  With the
-// layered scheme layer lo-d is A^d applied to the first fluid layer, A the diagonal
+// The same fill in one launch for walls of at most R (<= 4) layers (any depth with the
+// simple scheme, which reads the first fluid layer only).  With the layered scheme layer lo-d is A^d applied to the first fluid layer, A the diagonal
 // average above, so a 16 x 16 tile of columns needs the fluid layer on the tile
 // plus a halo of R columns.  The workgroup stages that patch in LDS and recomputes
 // the layers on shrinking patches with the same arithmetic (including the rounding
@@ -1162,10 +1162,12 @@ hipError_t launch_wall(cpmp_ctx *c) {
         if (P.wall_scheme == 2)   // ChemBoundaryComplex: one launch per level, as the reference
             for (int p = 0; p < passes; ++p)
                 hipLaunchKernelGGL(k_wall<TS>, g, dim3(TPB), 0, c->stream, P, rho, mu, c->mu_w, p);
-        else if (passes == 1) hipLaunchKernelGGL((k_wall_tile<1, TS>), gt, bt, 0, c->stream, P, rho, mu, c->mu_w);
+        else if (passes == 1 || P.wall_scheme == 0)   // simple scheme: any depth from the first fluid layer
+            hipLaunchKernelGGL((k_wall_tile<1, TS>), gt, bt, 0, c->stream, P, rho, mu, c->mu_w);
         else if (passes == 2) hipLaunchKernelGGL((k_wall_tile<2, TS>), gt, bt, 0, c->stream, P, rho, mu, c->mu_w);
         else if (passes == 3) hipLaunchKernelGGL((k_wall_tile<3, TS>), gt, bt, 0, c->stream, P, rho, mu, c->mu_w);
-        else   // deeper walls: one launch per layer
+        else if (passes == 4) hipLaunchKernelGGL((k_wall_tile<4, TS>), gt, bt, 0, c->stream, P, rho, mu, c->mu_w);
+        else   // deeper walls: one launch per layer (5 us each; the tile launch takes 5 to 7 us in all)
             for (int p = 0; p < passes; ++p)
                 hipLaunchKernelGGL(k_wall<TS>, g, dim3(TPB), 0, c->stream, P, rho, mu, c->mu_w, p);
         return hipGetLastError();
