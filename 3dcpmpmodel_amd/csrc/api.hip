@@ -267,11 +267,10 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
         return set_error(code, "allocation of %s failed", what);
     };
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) { delete c; return set_error(CPMP_EHIP, "stream"); }
-    const size_t popset = (size_t)c->N * 19 * c->pop_bytes;
-    if (hipMalloc(&c->f[0], popset) != hipSuccess) return fail(CPMP_ENOMEM, "populations A");
-    if (hipMalloc(&c->f[1], popset) != hipSuccess) return fail(CPMP_ENOMEM, "populations B");
-    if (hipMalloc(&c->rho, c->N * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "rho");
-    if (hipMalloc(&c->mu, c->N * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "mu");
+    const size_t popset = (size_t)c->N * 19 * c->pop_bytes, scal = (size_t)c->N * c->scal_bytes;
+    // the buffers, carved from one allocation
+    struct Part { void **p; size_t n; };
+    std::vector<Part> parts = {{&c->f[0], popset}, {&c->f[1], popset}, {&c->rho, scal}, {&c->mu, scal}};
     const char *fuse = std::getenv("CPMP_FUSE");
     size_t ring_elems = 0, chunk_elems = 0;
     const bool fuse_off = fuse && std::strcmp(fuse, "0") == 0;
@@ -281,34 +280,42 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
     if (c->moments) {
         c->collide_v1 = false;
         c->step_chunk = moment_chunk(p->nx, p->ny, p->nz, p->form);
-        if (hipMalloc(&c->rho_next, c->N * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "next rho");
-        if (hipMalloc(&c->mom, mset) != hipSuccess) return fail(CPMP_ENOMEM, "moments");
-        c->fuse_bytes = (size_t)c->N * c->scal_bytes + mset;
+        parts.push_back({&c->mom, mset});
+        c->fuse_bytes += mset;
     }
     // the population march sums the density inside the collide where the tiles cover the
     // lattice (not the one-thread-per-node collide of small FP64 lattices).  The adjoint of
     // the FP32 form runs it also where runs of steps take the moments.
-    if (!c->collide_v1 && !fuse_off && covered && (!c->moments || c->form == CPMP_FORM_FP32)) {
-        if (!c->rho_next && hipMalloc(&c->rho_next, c->N * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "next rho");
-        if (hipMalloc(&c->rbuf, ring_elems * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "tile rings");
-        if (hipMalloc(&c->cbuf, chunk_elems * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "chunk planes");
-        c->fuse_bytes = ((size_t)c->N + ring_elems + chunk_elems) * c->scal_bytes + (c->mom ? mset : 0);
+    const bool fused = !c->collide_v1 && !fuse_off && covered && (!c->moments || c->form == CPMP_FORM_FP32);
+    if (fused) {
+        parts.push_back({&c->rbuf, ring_elems * c->scal_bytes});
+        parts.push_back({&c->cbuf, chunk_elems * c->scal_bytes});
+        c->fuse_bytes += (ring_elems + chunk_elems) * c->scal_bytes;
+    }
+    // both double-buffer the density, and so does the FP16 form on every lattice: the
+    // previous density is the reference its populations are shifted by
+    if (c->moments || fused || c->form == CPMP_FORM_FP16) {
+        parts.push_back({&c->rho_next, scal});
+        c->fuse_bytes += scal;
     }
     if (covered && !fuse_off && !c->collide_v1) {   // populations tile-contiguous (pop_site)
         c->dp.tiled = 1;
         c->dp.nty = p->ny / kTileY;
         c->dp.ntz = p->nz / kTileZ;
     }
-    // the FP16 form double-buffers the density on every lattice: the previous
-    // density is the reference its populations are shifted by
-    if (c->form == CPMP_FORM_FP16 && !c->rho_next) {
-        if (hipMalloc(&c->rho_next, c->N * c->scal_bytes) != hipSuccess) return fail(CPMP_ENOMEM, "previous rho");
-        c->fuse_bytes = (size_t)c->N * c->scal_bytes;
+    parts.push_back({(void **)&c->mv, 3 * (size_t)c->N * sizeof(double)});
+    parts.push_back({(void **)&c->mu_w, 2 * (size_t)c->NXY * sizeof(double)});
+    parts.push_back({(void **)&c->red, reduce_scratch_doubles() * sizeof(double)});
+    parts.push_back({(void **)&c->staging, (size_t)c->N * sizeof(double)});
+    auto padded = [](size_t n) { return n < ((size_t)1 << 20) ? (n + 255) / 256 * 256 : (n + 65535) / 65536 * 65536; };
+    size_t total = 0;
+    for (const Part &w : parts) total += padded(w.n);
+    if (hipMalloc((void **)&c->block, total) != hipSuccess) return fail(CPMP_ENOMEM, "the lattice's buffers");
+    size_t at = 0;
+    for (const Part &w : parts) {
+        *w.p = c->block + at;
+        at += padded(w.n);
     }
-    if (hipMalloc((void **)&c->mv, 3 * c->N * sizeof(double)) != hipSuccess) return fail(CPMP_ENOMEM, "MV");
-    if (hipMalloc((void **)&c->mu_w, 2 * c->NXY * sizeof(double)) != hipSuccess) return fail(CPMP_ENOMEM, "wall mu");
-    if (hipMalloc((void **)&c->red, reduce_scratch_doubles() * sizeof(double)) != hipSuccess) return fail(CPMP_ENOMEM, "reduce");
-    if (hipMalloc((void **)&c->staging, c->N * sizeof(double)) != hipSuccess) return fail(CPMP_ENOMEM, "staging");
     if (hipMemsetAsync(c->f[0], 0, popset, c->stream) != hipSuccess || hipMemsetAsync(c->f[1], 0, popset, c->stream) != hipSuccess ||
         hipMemsetAsync(c->rho, 0, c->N * c->scal_bytes, c->stream) != hipSuccess ||
         hipMemsetAsync(c->mu, 0, c->N * c->scal_bytes, c->stream) != hipSuccess ||
@@ -324,9 +331,8 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
 int cpmp_destroy(cpmp_ctx *c) {
     if (!c) return CPMP_OK;
     if (c->stream) { hipSetDevice(c->p.device); hipStreamSynchronize(c->stream); }
-    for (void *ptr : {c->f[0], c->f[1], c->rho, c->rho_next, c->rbuf, c->cbuf, c->mom, c->mu, (void *)c->mv, (void *)c->mu_w,
-                      (void *)c->red, (void *)c->staging, (void *)c->adj_ws})
-        if (ptr) hipFree(ptr);
+    if (c->block) hipFree(c->block);
+    if (c->adj_ws) hipFree(c->adj_ws);
     if (c->timers) {
         for (auto &e : c->timers->ev) if (e) hipEventDestroy(e);
         delete c->timers;

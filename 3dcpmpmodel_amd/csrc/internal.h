@@ -54,6 +54,7 @@ struct cpmp_ctx {
     size_t pop_bytes = 0;       // bytes of one population value
     size_t scal_bytes = 0;      // bytes of one rho/mu value
     hipStream_t stream = nullptr;
+    char *block = nullptr;      // the allocation that holds every buffer below but adj_ws
     void *f[2] = {nullptr, nullptr};
     int cur = 0;
     void *rho = nullptr, *mu = nullptr;
