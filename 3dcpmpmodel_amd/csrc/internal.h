@@ -100,11 +100,12 @@ int march_chunk(int nx, int ny, int nz, int form);
 bool node_collide(int nx, int ny, int nz, int form);
 // runs of steps hand 12 moments per node and the density from one step to the next
 // (the reference's unit rates; not the FP16 form, whose state is defined by its stored
-// populations).  Lattices below 100 000 nodes keep the population kernels: there a step
-// is a few launches' latency, and the march takes longer from end to end than a launch of
-// one thread per node (us per step, population kernels against moments: 64x1x32 FP64
-// 19.0 / 20.1, 32^3 FP64 17.6 / 22.1, 48x40x36 FP32 27.9 / 30.9; 64^3 FP64 40.2 / 35.9,
-// FP32 34.5 / 30.5, 96x96x64 FP32 65.9 / 47.6).  CPMP_COLLIDE=march or CPMP_XC take the
+// populations).  Lattices below 80 000 nodes keep the population kernels: there a step is
+// a few launches' latency, and the march takes longer from end to end than a launch of one
+// thread per node (us per step, population kernels against moments: 32^3 FP64 15.8 / 19.3,
+// 48x40x36 FP32 23.8 / 26.0, FP64 26.8 / 29.2; 44x45x46 FP32 22.3 / 20.7, FP64 26.3 / 23.5).
+// One-row FP32 lattices take the moments at any size: the population march of this form
+// fills 1 of 8 lanes there (300x1x100 27.5 / 17.5).  CPMP_COLLIDE=march or CPMP_XC take the
 // moments on any lattice; CPMP_COLLIDE=v1 and, on lattices the march tiles cover,
 // CPMP_FUSE=0 keep the populations.
 bool moment_path(const cpmp_params &p, const DevParams &d, bool fuse_off, bool covered);

@@ -1236,7 +1236,7 @@ template <class TS> static const TS *ref_buffer(const cpmp_ctx *c) {
 bool moment_path(const cpmp_params &p, const DevParams &d, bool fuse_off, bool covered) {
     const char *e = std::getenv("CPMP_COLLIDE");
     if (!d.unit_rates || p.form == CPMP_FORM_FP16 || (e && std::strcmp(e, "v1") == 0) || (fuse_off && covered)) return false;
-    return d.N >= 100000 || (e && std::strcmp(e, "march") == 0) || std::getenv("CPMP_XC");
+    return d.N >= 80000 || (p.ny == 1 && p.form == CPMP_FORM_FP32) || (e && std::strcmp(e, "march") == 0) || std::getenv("CPMP_XC");
 }
 
 hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool last) {

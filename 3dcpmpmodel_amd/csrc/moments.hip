@@ -145,7 +145,15 @@ enum { kPlain, kQp, kGuo };   // force term: exact difference, with Qp, Guo (Qp 
 // arrives: after the plane behind it has collided, a node holds its 19 pulled values and
 // writes their moments (OUT_P: its post-collision populations too).  Nothing is exchanged between workgroups within a
 // step, so any lattice size works and no density completion follows; the price is the
-// ring: 340 collisions for 256 nodes, and two more planes per chunk.
+// ring: 476 collisions for 384 nodes, and two more planes per chunk.
+//
+// Bound: memory.  At 256^3 FP32 a launch moves 2.18 GB (1.74 GB of state) in 0.453 ms, 4.8
+// TB/s, what a large copy reaches; the VALU is busy 71 % of it.  FP64 0.89 ms, 4.7 TB/s.  The
+// population march with its density completion took 0.62 (FP32) and 1.24 ms (FP64).
+// Tile: 12 x 32 fills 8 waves, 2 per SIMD, and two workgroups a CU (8 x 32: 5.3 waves
+// unevenly over the SIMDs, step 0.623 against 0.604 ms at 256^3 FP32; 12 x 64 with one
+// workgroup of 15 waves per CU 0.568 against 0.579, but its tail grows on other sizes).
+// 4 waves per SIMD (128 VGPRs) keep the second workgroup: at 136 the step took 0.689 ms.
 template <class TF, class TS, class TC, class TL, bool IN_P, bool OUT_P, bool DIAG, bool NW, int FC>
 __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 ? 4 : 2) k_moment_step(const DevParams P, const StepArgs<TF, TS, TC> A) {
     __shared__ Pair<TC> s_rm[7][TL::EP];       // planes x-3 .. x+3
@@ -338,7 +346,13 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 ? 4 : 2) k_moment_step
             if (own && x >= xa && x < xb) {
                 const unsigned b = (unsigned)x * (unsigned)pl + psite;
 #pragma unroll
-                for (int q = 0; q < Q; ++q) __builtin_nontemporal_store((TF)out[q], &A.fout[(unsigned)q * (unsigned)P.N + b]);
+                for (int q = 0; q < Q; ++q) {
+                    // whole lines in the tiled layout; elsewhere the L2 has to merge them
+                    // (150x117x83: 136 us a step with streaming stores, 79 without)
+                    TF *p = &A.fout[(unsigned)q * (unsigned)P.N + b];
+                    if (P.tiled) __builtin_nontemporal_store((TF)out[q], p);
+                    else *p = (TF)out[q];
+                }
             }
         }
         __syncthreads();                       // mailbox of plane x posted, plane x - 3 no longer read
@@ -459,7 +473,9 @@ hipError_t launch_form(cpmp_ctx *c, bool in_p, bool out_p, double *mv, TS *uout)
 // Planes per workgroup.  A chunk of n planes collides n + 2 and loads 7 planes of rho and
 // mu before its first (together about 4 planes' time), and the launch takes as many
 // rounds as its workgroups need places on the device (2 per CU with 4-byte arithmetic,
-// 1 with 8-byte: LDS), so the chunk count that minimises rounds * (n + 4) is taken.
+// 1 with 8-byte: LDS), so the chunk length that minimises rounds * (n + 4) is taken.  Within
+// 3 % of the best of a sweep over 1..24 planes on 13 lattices (64^3 FP64 4: 36.5 us, 8: 54.6;
+// 128^3 FP32 11: 87.5, 4: 104, 24: 134; 256^3 FP32 32: 533, 43: 568).
 // CPMP_XC overrides.
 int moment_chunk(int nx, int ny, int nz, int form) {
     if (const char *e = std::getenv("CPMP_XC")) {

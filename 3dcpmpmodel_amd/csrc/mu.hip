@@ -114,6 +114,11 @@ __device__ __forceinline__ TS mu_node(const DevParams &P, Get get) {
 // values along x stay in registers, the in-plane neighbours are read through the L1 (their
 // lines are the ones neighbouring lanes and waves read), each one plane ahead.  Columns
 // are numbered y * nz + z, so every lattice, one row in y included, fills its waves.
+// Bound: latency and VALU (256^3 FP32 75 us, 43 us of it VALU; FP64 129 us against 56 us of
+// traffic).  An LDS ring per 8 x 32 tile with a barrier a plane took 63 us and 8 us for its
+// list of interface nodes there, but 152 us in FP64 (112 with ln64), 67 us against 19 on
+// 3001 x 1 x 501 and 19 against 16 on 150 x 117 x 83; two nodes per thread, read as pairs,
+// made the FP32 step 1 % slower.
 // H: radius of the Laplacian, 2 (5 points) or 3 (7 points).  rho_solid (if given) receives
 // the wall density of solid nodes, rho_copy (if given) the density of every node.
 template <class TS, int H>

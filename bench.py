@@ -17,6 +17,9 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_HBM_GBS = 8000.0     # MI355X HBM3E, AMD published
+# bytes per node that a step within a run reads and writes of the state: 13 numbers (density
+# and 12 moments) each way in the precision they are computed in; FP16 storage: 19 populations
+STATE_BYTES = {"fp64": 2 * 13 * 8, "fp32": 2 * 13 * 4, "fp32a": 2 * 13 * 4, "fp16": 2 * 19 * 2}
 G_RKE, L_RKE = 0.0319804, 8.25467   # CoCurve_RKE_2.txt Tr=0.60 row times Rc
 
 
@@ -42,7 +45,7 @@ def time_form(cpmp, n, form, steps, warmup):
     dt = time.perf_counter() - t0
     s = g.reduce()
     ktimes, per = g.kernel_times(max(5, min(20, steps // 10)))
-    bpn = g.algorithmic_bytes_per_node()
+    bpn = STATE_BYTES[form]
     g.close()
     nodes = n ** 3
     return dict(ms_per_step=dt / steps * 1e3, mlups=nodes * steps / dt / 1e6, kernel_ms=ktimes, launches=per,
@@ -294,7 +297,7 @@ def large_run(cpmp, fwd_steps=10000, adj_steps=2000, every=100):
     t_plain = time.perf_counter() - t0
     ktimes, _ = lat.kernel_times(kt_steps)
     mlups = nodes * (n_plain - kt_steps) / t_plain / 1e6
-    bpn = lat.algorithmic_bytes_per_node()
+    bpn = STATE_BYTES["fp32"]
     s = lat.reduce()
     log(f"[large] {mlups:.1f} MLUPS, kernels {ktimes}, mass {s.mass:.6e}")
     target = lat.get("rho")
@@ -453,8 +456,8 @@ def main():
     achieved = main_form["bytes_per_node"] * nodes / (kc * 1e-3) / 1e9
     roofline = dict(bound="hbm", achieved=round(achieved, 1), peak=PEAK_HBM_GBS, unit="GB/s",
                     frac=round(achieved / PEAK_HBM_GBS, 4),
-                    traffic=measured_traffic("k_collide_march_fp32") if n == 256 else None,
-                    kernel="k_collide_march (fp32)", bytes_per_node=main_form["bytes_per_node"])
+                    traffic=measured_traffic("k_moment_step_fp32") if n == 256 else None,
+                    kernel="k_moment_step (fp32)", bytes_per_node=main_form["bytes_per_node"])
     step_bw = main_form["bytes_per_node"] * nodes / (main_form["ms_per_step"] * 1e-3) / 1e9
     acc = adj = None
     if not args.no_accuracy:
@@ -499,7 +502,7 @@ def main():
         "roofline": roofline,
         "step_roofline_frac": round(step_bw / PEAK_HBM_GBS, 4),
         # per form: the collide's and the step's fraction of the 8 TB/s roofline at the
-        # form's algorithmic population bytes (2 x 19 x storage size per node)
+        # bytes of the state that the form carries from step to step (STATE_BYTES)
         "forms": {k: {"mlups": round(v["mlups"], 1), "ms_per_step": round(v["ms_per_step"], 4),
                       "kernel_ms": {a: round(b, 4) for a, b in v["kernel_ms"].items()},
                       "bytes_per_node": v["bytes_per_node"], "mass_drift": v["mass_drift"],
