@@ -276,7 +276,8 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
     const bool fuse_off = fuse && std::strcmp(fuse, "0") == 0;
     const bool covered = fuse_geometry(p->nx, p->ny, p->nz, c->dp.xc, &ring_elems, &chunk_elems);
     const size_t mset = moment_bytes(p->nx, p->ny, p->nz, p->form);
-    c->moments = mset <= popset && moment_path(*p, c->dp, fuse_off, covered);
+    // (the kernel addresses a plane of a set with 32-bit offsets)
+    c->moments = mset <= popset && mset / (size_t)p->nx < ((size_t)1 << 32) && moment_path(*p, c->dp, fuse_off, covered);
     if (c->moments) {
         c->collide_v1 = false;
         c->step_chunk = moment_chunk(p->nx, p->ny, p->nz, p->form);

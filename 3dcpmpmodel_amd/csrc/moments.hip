@@ -473,7 +473,7 @@ hipError_t launch_form(cpmp_ctx *c, bool in_p, bool out_p, double *mv, TS *uout)
 // Planes per workgroup.  A chunk of n planes collides n + 2 and loads 7 planes of rho and
 // mu before its first (together about 4 planes' time), and the launch takes as many
 // rounds as its workgroups need places on the device (2 per CU with 4-byte arithmetic,
-// 1 with 8-byte: LDS), so the chunk length that minimises rounds * (n + 4) is taken.  Within
+// 1 with 8-byte: LDS; twice as many of the one-row tiles' 4 waves), so the chunk length that minimises rounds * (n + 4) is taken.  Within
 // 3 % of the best of a sweep over 1..24 planes on 13 lattices (64^3 FP64 4: 36.5 us, 8: 54.6;
 // 128^3 FP32 11: 87.5, 4: 104, 24: 134; 256^3 FP32 32: 533, 43: 568).
 // CPMP_XC overrides.
@@ -485,7 +485,7 @@ int moment_chunk(int nx, int ny, int nz, int form) {
     const bool flat = ny == 1;
     const int ty = 12;
     const long long tiles = flat ? (nz + 191) / 192 : (long long)((ny + ty - 1) / ty) * ((nz + 31) / 32);
-    const long long places = form == CPMP_FORM_FP64 ? 256 : 512;
+    const long long places = (form == CPMP_FORM_FP64 ? 256 : 512) * (flat ? 2 : 1);
     int best = 32;
     double cost = 1e300;
     for (int n = 1; n <= 128; ++n) {
