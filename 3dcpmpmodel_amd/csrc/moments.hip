@@ -384,7 +384,17 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 ? 4 : 2) k_moment_step
                     __builtin_nontemporal_store(v, lane_at(b + (size_t)k * pl, site));
                     if (edge) s_edge[k * TL::TY + eslot] = v;
                 }
-                if (fluid) *lane_at(A.rho_out + (size_t)xp * pl, node) = (TS)n[0];
+                if (fluid) {
+                    // FP32 arithmetic on FP64 storage: the density is summed in its own
+                    // precision
+                    TS d = (TS)n[0];
+                    if constexpr (sizeof(TS) > sizeof(TC)) {
+                        d = (TS)fa[0];
+#pragma unroll
+                        for (int q = 1; q < Q; ++q) d += (TS)fa[q];
+                    }
+                    *lane_at(A.rho_out + (size_t)xp * pl, node) = d;
+                }
             }
             // keeps the other arrivals out of the registers that the moments need
             __builtin_amdgcn_sched_barrier(0);

@@ -91,3 +91,19 @@ def test_moment_runs_split_into_calls_are_bitwise_the_same(cpmp, monkeypatch, tm
         assert np.array_equal(a.get(field), c.get(field)), field
     for g in (a, b, c):
         g.close()
+
+
+@pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[10]], ids=lambda c: "x".join(map(str, c[0])))
+def test_fp32_arithmetic_form_sums_the_density_in_fp64(cpmp, monkeypatch, case):
+    """FP64 storage with FP32 arithmetic: the stored density is the FP64 sum of the 19
+    values that the next step pulls, whichever step of a call wrote it.  Two sums of 19
+    terms in any order differ by at most 2 * 18 * 2^-53 of the sum of magnitudes."""
+    a = lattice(cpmp, monkeypatch, case, "fp32a", "march")
+    fluid = a.get("type") == 1
+    for n in (1, 4):
+        a.step(n)
+        f = a.get("f").reshape(19, -1)[:, fluid]
+        err = np.max(np.abs(a.get("rho")[fluid] - f.sum(axis=0)) / np.abs(f).sum(axis=0))
+        print(f"[moments] {case[0]} fp32a density: {err:.2e}", flush=True)
+        assert err <= 36 * 2.0 ** -53
+    a.close()
