@@ -1234,9 +1234,11 @@ template <class TS> static const TS *ref_buffer(const cpmp_ctx *c) {
 }
 
 bool moment_path(const cpmp_params &p, const DevParams &d, bool fuse_off, bool covered) {
+    if (!d.unit_rates || p.form == CPMP_FORM_FP16) return false;
     const char *e = std::getenv("CPMP_COLLIDE");
-    if (!d.unit_rates || p.form == CPMP_FORM_FP16 || (e && std::strcmp(e, "v1") == 0) || (fuse_off && covered)) return false;
-    return d.N >= 80000 || (p.ny == 1 && p.form == CPMP_FORM_FP32) || (e && std::strcmp(e, "march") == 0) || std::getenv("CPMP_XC");
+    if (e && std::strcmp(e, "moments") == 0) return true;
+    if ((e && (std::strcmp(e, "v1") == 0 || std::strcmp(e, "march") == 0)) || (fuse_off && covered)) return false;
+    return d.N >= 80000 || (p.ny == 1 && p.form == CPMP_FORM_FP32);
 }
 
 hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool last) {
@@ -1307,8 +1309,8 @@ hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool last) {
             using T1 = std::true_type;
             using F0 = std::false_type;
             const bool ur = c->dp.unit_rates != 0;
-            // FP64 storage sums the density here with general rates only (the unit-rate
-            // lattices take the moments)
+            // FP64 storage sums the density here with the general-rate collision only
+            // (unit-rate lattices take the moments unless CPMP_COLLIDE=march)
             if (rs) {
                 if constexpr (std::is_same<TF, double>::value) {
                     if (want_mv) go(T1{}, T1{}, F0{}); else go(F0{}, T1{}, F0{});

@@ -57,7 +57,7 @@ def test_moment_runs_match_the_population_kernels(cpmp, monkeypatch, case, form,
     taken from a wrong node shows at once).  A step sums 19 values and the moments once
     more, some 40 roundings of at most the largest population: 7 * 40 * 2^-53 = 3e-14
     (FP64) and 1.7e-5 / 2 (FP32) relative to the density, and smaller in practice."""
-    a = lattice(cpmp, monkeypatch, case, form, "march")
+    a = lattice(cpmp, monkeypatch, case, form, "moments")
     b = lattice(cpmp, monkeypatch, case, form, "v1")
     a.step(7)
     b.step(7)
@@ -77,9 +77,9 @@ def test_moment_runs_match_the_population_kernels(cpmp, monkeypatch, case, form,
 def test_moment_runs_split_into_calls_are_bitwise_the_same(cpmp, monkeypatch, tmp_path, case, form):
     """the populations between calls lose nothing: one call of 6 steps, and calls of
     1 + 2 + 3 steps with a checkpoint taken into another lattice in between"""
-    a = lattice(cpmp, monkeypatch, case, form, "march")
-    b = lattice(cpmp, monkeypatch, case, form, "march")
-    c = lattice(cpmp, monkeypatch, case, form, "march")
+    a = lattice(cpmp, monkeypatch, case, form, "moments")
+    b = lattice(cpmp, monkeypatch, case, form, "moments")
+    c = lattice(cpmp, monkeypatch, case, form, "moments")
     a.step(6)
     b.step(1)
     b.step(2)
@@ -98,7 +98,7 @@ def test_fp32_arithmetic_form_sums_the_density_in_fp64(cpmp, monkeypatch, case):
     """FP64 storage with FP32 arithmetic: the stored density is the FP64 sum of the 19
     values that the next step pulls, whichever step of a call wrote it.  Two sums of 19
     terms in any order differ by at most 2 * 18 * 2^-53 of the sum of magnitudes."""
-    a = lattice(cpmp, monkeypatch, case, "fp32a", "march")
+    a = lattice(cpmp, monkeypatch, case, "fp32a", "moments")
     fluid = a.get("type") == 1
     for n in (1, 4):
         a.step(n)
@@ -107,3 +107,26 @@ def test_fp32_arithmetic_form_sums_the_density_in_fp64(cpmp, monkeypatch, case):
         print(f"[moments] {case[0]} fp32a density: {err:.2e}", flush=True)
         assert err <= 36 * 2.0 ** -53
     a.close()
+
+
+@pytest.mark.parametrize("form", ["fp64", "fp32", "fp32a"])
+def test_the_switches_select_the_path(cpmp, monkeypatch, form):
+    """CPMP_COLLIDE=moments takes the moments on a lattice of any size, =march the population
+    march, and CPMP_XC changes the chunk only: told apart by the moment set, 12 values per
+    node and more, in the lattice's memory"""
+    dims, n, word = (64, 16, 64), 64 * 16 * 64, 8 if form == "fp64" else 4
+
+    def memory(collide, xc):
+        for k, v in (("CPMP_COLLIDE", collide), ("CPMP_XC", xc)):
+            monkeypatch.setenv(k, v) if v else monkeypatch.delenv(k, raising=False)
+        g = cpmp.Lattice(cpmp.make_params(*dims, eos="RKE", tr=0.6, nwall=0, form=form))
+        b = g.memory()
+        g.close()
+        return b
+
+    monkeypatch.delenv("CPMP_FUSE", raising=False)
+    v1 = memory("v1", None)
+    assert memory("moments", None) - v1 >= 12 * word * n
+    assert memory("moments", "4") - v1 >= 12 * word * n
+    assert memory("march", "4") - v1 < 12 * word * n
+    assert memory(None, "4") - v1 < 12 * word * n
