@@ -105,7 +105,8 @@ bool node_collide(int nx, int ny, int nz, int form);
 // thread per node (us per step, population kernels against moments: 32^3 FP64 15.8 / 19.3,
 // 48x40x36 FP32 23.8 / 26.0, FP64 26.8 / 29.2; 44x45x46 FP32 22.3 / 20.7, FP64 26.3 / 23.5).
 // One-row FP32 lattices take the moments at any size: the population march of this form
-// fills 1 of 8 lanes there (300x1x100 27.5 / 17.5).  CPMP_COLLIDE=moments takes the moments
+// fills 1 of 8 lanes there (300x1x100 27.5 / 17.5).  Some lattices of 1 plane or 2 to 4 rows
+// keep the populations at any size (thin_lattice).  CPMP_COLLIDE=moments takes the moments
 // on a lattice of any size; CPMP_COLLIDE=v1 or march and, on lattices the march tiles cover,
 // CPMP_FUSE=0 keep the populations.  The moment sets alternate with the population sets, so
 // a lattice whose moment set is larger (edge columns of tiles a few nodes wide) keeps the

@@ -1199,11 +1199,7 @@ bool fuse_geometry(int nx, int ny, int nz, int xc, size_t *ring_elems, size_t *c
 // workgroups) takes chunks of 4, 8 % faster than single planes in FP32 and FP16
 // (FP64 lattices below 2048 workgroups of 2 planes take the per-node collide
 // instead, node_collide).  CPMP_XC overrides.
-int march_chunk(int nx, int ny, int nz, int form) {
-    if (const char *e = std::getenv("CPMP_XC")) {
-        const int v = std::atoi(e);
-        if (v >= 1 && v <= MXC) return v;
-    }
+static int march_chunk_rule(int nx, int ny, int nz, int form) {
     const long long tiles = (long long)((ny + MTY - 1) / MTY) * ((nz + MTZ - 1) / MTZ);
     if (!fp64_storage(form) && (long long)((nx + 1) / 2) * tiles < 2048) return 1;   // small lattice
     for (int c = MXC; c >= 2; c /= 2)
@@ -1213,6 +1209,13 @@ int march_chunk(int nx, int ny, int nz, int form) {
     for (int c = MXC; c >= 2; c /= 2)
         if ((nx + c - 1) / c * tiles >= 1024) return c;
     return 2;
+}
+int march_chunk(int nx, int ny, int nz, int form) {
+    if (const char *e = std::getenv("CPMP_XC")) {
+        const int v = std::atoi(e);
+        if (v >= 1 && v <= MXC) return v;
+    }
+    return march_chunk_rule(nx, ny, nz, form);
 }
 bool density_fused(const cpmp_ctx *c) { return c->rbuf && !c->collide_v1 && !c->moments; }
 
@@ -1233,12 +1236,40 @@ template <class TS> static const TS *ref_buffer(const cpmp_ctx *c) {
     return c->form == CPMP_FORM_FP16 ? (const TS *)c->rho_next : nullptr;
 }
 
+// Thin lattices of 80 000 nodes and more that the population kernels step faster than the
+// moments do: the 12 x 32 tile repeats the periodic rows of ny = 2..4 in most of its lanes.
+// us per call of 20 steps, population kernels against moments.
+static bool thin_lattice(const cpmp_params &p) {
+    const bool node = node_collide(p.nx, p.ny, p.nz, p.form);
+    const long long n = (long long)p.nx * p.ny * p.nz;
+    auto up = [](long long a, long long b) { return (a + b - 1) / b; };
+    if (p.form == CPMP_FORM_FP64) {
+        // one plane: three collided for one stepped, and the places of FP64 (256 workgroups) hold
+        // one round (1x146x582 493 / 417, 1x300x400 602 / 675, 1x700x700 1428 / 1876)
+        if (p.nx == 1) return up(p.ny, 12) * up(p.nz, 32) > 256;
+        // against one thread per node, in lanes of its 4 x 64 blocks (428x2x225 878 / 1300, 922x3x36
+        // 672 / 849, 575x3x97 820 / 971, 1930x4x34 1252 / 1470; 981x3x70 1191 / 1164, 2.25 times the
+        // lanes; 300x5x60 597 / 538)
+        const long long lanes = up(p.ny, 12) * 12 * up(p.nz, 32) * 32, node_lanes = up(p.ny, 4) * 4 * up(p.nz, 64) * 64;
+        if (node) return p.ny == 2 || (p.ny <= 4 && 2 * lanes >= 5 * node_lanes);
+        // against the population march with long chunks (496x2x1368, 16 planes: 6776 / 6973;
+        // 295x2x1311, 8 planes: 3986 / 3888)
+        return p.ny == 2 && march_chunk_rule(p.nx, p.ny, p.nz, p.form) >= 16;
+    }
+    if (p.ny != 2) return false;
+    // 544x2x83 607 / 654, 40x2x1267 598 / 643; 489x2x197 1178 / 890
+    if (p.form == CPMP_FORM_FP32A) return node && n < 160000;
+    // march chunks of 4 and more: 496x2x1368 2968 / 3518, 212x2x1264 1486 / 1580; of 2: 562x2x996 0.80
+    // of the time; of 1: 100x2x1067 1189 / 816
+    return march_chunk_rule(p.nx, p.ny, p.nz, p.form) >= 4;
+}
+
 bool moment_path(const cpmp_params &p, const DevParams &d, bool fuse_off, bool covered) {
     if (!d.unit_rates || p.form == CPMP_FORM_FP16) return false;
     const char *e = std::getenv("CPMP_COLLIDE");
     if (e && std::strcmp(e, "moments") == 0) return true;
     if ((e && (std::strcmp(e, "v1") == 0 || std::strcmp(e, "march") == 0)) || (fuse_off && covered)) return false;
-    return d.N >= 80000 || (p.ny == 1 && p.form == CPMP_FORM_FP32);
+    return (d.N >= 80000 && !thin_lattice(p)) || (p.ny == 1 && p.form == CPMP_FORM_FP32);
 }
 
 hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool last) {

@@ -27,6 +27,8 @@ CASES = [
     ((12, 13, 34), 5, 3, dict(K1=0.003, K2=-0.003)),
     ((12, 23, 24), 5, 3, dict(forcing=1)),
     ((12, 13, 34), 5, 0, dict(forcing=1, K1=0.003, K2=-0.003)),
+    ((13, 2, 40), 5, 3, {}),                    # rows that are each other's neighbours on both sides
+    ((7, 4, 33), 3, 0, {}),
     ((20, 1, 191), 6, 3, {}),
     ((6, 1, 193), 1, 0, {}),
     ((11, 1, 385), 4, 3, dict(forcing=1)),
@@ -73,7 +75,7 @@ def test_moment_runs_match_the_population_kernels(cpmp, monkeypatch, case, form,
 
 
 @pytest.mark.parametrize("form", ["fp64", "fp32", "fp32a"])
-@pytest.mark.parametrize("case", [CASES[1], CASES[7], CASES[8], CASES[10]], ids=lambda c: "x".join(map(str, c[0])))
+@pytest.mark.parametrize("case", [CASES[1], CASES[7], CASES[8], CASES[10], CASES[12]], ids=lambda c: "x".join(map(str, c[0])))
 def test_moment_runs_split_into_calls_are_bitwise_the_same(cpmp, monkeypatch, tmp_path, case, form):
     """the populations between calls lose nothing: one call of 6 steps, and calls of
     1 + 2 + 3 steps with a checkpoint taken into another lattice in between"""
@@ -93,7 +95,7 @@ def test_moment_runs_split_into_calls_are_bitwise_the_same(cpmp, monkeypatch, tm
         g.close()
 
 
-@pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[10]], ids=lambda c: "x".join(map(str, c[0])))
+@pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[10], CASES[12]], ids=lambda c: "x".join(map(str, c[0])))
 def test_fp32_arithmetic_form_sums_the_density_in_fp64(cpmp, monkeypatch, case):
     """FP64 storage with FP32 arithmetic: the stored density is the FP64 sum of the 19
     values that the next step pulls, whichever step of a call wrote it.  Two sums of 19
@@ -130,3 +132,27 @@ def test_the_switches_select_the_path(cpmp, monkeypatch, form):
     assert memory("moments", "4") - v1 >= 12 * word * n
     assert memory("march", "4") - v1 < 12 * word * n
     assert memory(None, "4") - v1 < 12 * word * n
+
+
+@pytest.mark.parametrize("form,dims,moments", [
+    ("fp64", (428, 2, 225), False), ("fp64", (873, 2, 263), True), ("fp64", (496, 2, 1368), False),
+    ("fp64", (922, 3, 36), False), ("fp64", (981, 3, 70), True), ("fp64", (968, 4, 34), False),
+    ("fp64", (300, 5, 60), True), ("fp64", (1, 300, 400), False), ("fp64", (1, 146, 582), True),
+    ("fp32a", (544, 2, 83), False), ("fp32a", (489, 2, 197), True), ("fp32a", (922, 3, 36), True),
+    ("fp32", (212, 2, 1264), False), ("fp32", (562, 2, 996), True), ("fp32", (100, 2, 1067), True),
+])
+def test_thin_lattices_take_the_faster_path(cpmp, monkeypatch, form, dims, moments):
+    """lattices of one plane or of 2 to 4 rows on both sides of the rule; the moment set, 12
+    values per node and more, shows in the lattice's memory"""
+    n, word = dims[0] * dims[1] * dims[2], 8 if form == "fp64" else 4
+
+    def memory(collide):
+        monkeypatch.setenv("CPMP_COLLIDE", collide) if collide else monkeypatch.delenv("CPMP_COLLIDE", raising=False)
+        g = cpmp.Lattice(cpmp.make_params(*dims, eos="RKE", tr=0.6, nwall=0, form=form))
+        b = g.memory()
+        g.close()
+        return b
+
+    monkeypatch.delenv("CPMP_FUSE", raising=False)
+    monkeypatch.delenv("CPMP_XC", raising=False)
+    assert (memory(None) - memory("v1") >= 12 * word * n) == moments
