@@ -262,6 +262,7 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
     c->scal_bytes = scal_size(p->form);
     fill_devparams(c);
     c->collide_v1 = node_collide(p->nx, p->ny, p->nz, p->form);
+    c->mu_chunk = mu_march_chunk(p->nx, p->ny, p->nz, p->form);
     auto fail = [&](int code, const char *what) {
         cpmp_destroy(c);
         return set_error(code, "allocation of %s failed", what);

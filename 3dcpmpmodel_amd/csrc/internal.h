@@ -64,6 +64,7 @@ struct cpmp_ctx {
     bool collide_v1 = false;    // one-thread-per-node collide (node_collide)
     bool moments = false;       // runs of steps carry 13 moments per node (moment_path)
     int step_chunk = 0;         // x planes per workgroup of the moment step
+    int mu_chunk = 0;           // x planes per workgroup of the chemical-potential march (0: by columns)
     // a moment set; the population set that is not current holds the other.  mom_at: which
     // one holds the moments of the current populations (0 none, 1 mom, 2 the population set)
     void *mom = nullptr;
@@ -93,6 +94,7 @@ bool density_fused(const cpmp_ctx *c);
 bool fuse_geometry(int nx, int ny, int nz, int xc, size_t *ring_elems, size_t *chunk_elems);
 // forms whose populations, rho and mu are stored in FP64 (FP64, FP32A)
 inline bool fp64_storage(int form) { return form == CPMP_FORM_FP64 || form == CPMP_FORM_FP32A; }
+int mu_march_chunk(int nx, int ny, int nz, int form);
 // x planes per march workgroup for a lattice and storage form (CPMP_XC overrides)
 int march_chunk(int nx, int ny, int nz, int form);
 // the one-thread-per-node collide instead of the x march (CPMP_COLLIDE=v1 / march

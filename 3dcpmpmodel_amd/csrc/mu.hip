@@ -4,6 +4,9 @@
 #include "device_common.h"
 
 #include <algorithm>
+#include <cstdlib>
+#include <cstring>
+#include <type_traits>
 
 namespace cpmp {
 
@@ -114,11 +117,10 @@ __device__ __forceinline__ TS mu_node(const DevParams &P, Get get) {
 // values along x stay in registers, the in-plane neighbours are read through the L1 (their
 // lines are the ones neighbouring lanes and waves read), each one plane ahead.  Columns
 // are numbered y * nz + z, so every lattice, one row in y included, fills its waves.
-// Bound: latency and VALU (256^3 FP32 75 us, 43 us of it VALU; FP64 129 us against 56 us of
-// traffic).  An LDS ring per 8 x 32 tile with a barrier a plane took 63 us and 8 us for its
-// list of interface nodes there, but 152 us in FP64 (112 with ln64), 67 us against 19 on
-// 3001 x 1 x 501 and 19 against 16 on 150 x 117 x 83; two nodes per thread, read as pairs,
-// made the FP32 step 1 % slower.
+// Bound: latency and VALU (256^3 FP64 129 us against 56 us of traffic; FP32 75 us, 43 us of it
+// VALU).  The LDS march below took 112 us in FP64 with a list of interface nodes apart (152 with
+// the library's logarithm), 36 us against 14 on 3001 x 1 x 501 and 17 against 15 on
+// 150 x 117 x 83; two nodes per thread, read as pairs, made the FP32 step 1 % slower.
 // H: radius of the Laplacian, 2 (5 points) or 3 (7 points).  rho_solid (if given) receives
 // the wall density of solid nodes, rho_copy (if given) the density of every node.
 template <class TS, int H>
@@ -177,12 +179,124 @@ __global__ void __launch_bounds__(TPB) k_mu_columns(const DevParams P, const TS 
     }
 }
 
+// The same as a march over 8 x 32 tiles: rho of planes x-H..x+H with an in-plane halo of H
+// sits in an LDS ring of 2H + 2 planes (the extra slot receives the plane entering the ring
+// while slower waves still read the one that left it, so one barrier a plane suffices), and
+// each rho value is fetched from memory about once per tile.  Two planes are in flight.
+// For large lattices of 4-byte densities, where the columns' reads past the L1 bound them
+// (512x512x256: 265 us, 209 here: 2.5 TB/s of the 536 MB it cannot do without).
+constexpr int kMuT = kTileY * kTileZ;
+template <class TS, int H>
+__global__ void __launch_bounds__(kMuT) k_mu_march(const DevParams P, const TS *__restrict__ rho, TS *__restrict__ mu,
+                                                   TS *__restrict__ rho_solid, TS *__restrict__ rho_copy, int xc, int ntz,
+                                                   int nty) {
+    constexpr int R = 2 * H + 2, LZ = kTileZ + 2 * H, LP = (kTileY + 2 * H) * LZ;
+    __shared__ TS s_rho[R][LP];
+    int t = blockIdx.x;
+    {   // each XCD takes a contiguous range of tiles, neighbours sharing an L2
+        const int n = gridDim.x, k = t & 7;
+        t = k * (n >> 3) + min(k, n & 7) + (t >> 3);
+    }
+    const int tzi = t % ntz;
+    t /= ntz;
+    const int y0 = t % nty * kTileY, z0 = tzi * kTileZ;
+    const int xa = t / nty * xc, xb = min(xa + xc, P.nx);
+    const int tid = threadIdx.x, ty = tid / kTileZ, tz = tid % kTileZ, y = y0 + ty, z = z0 + tz;
+    const bool inr = y < P.ny && z < P.nz, solid = is_solid(P, z);
+    const int pl = P.ny * P.nz;
+    constexpr int HE = (LP + kMuT - 1) / kMuT;
+    unsigned hoff[HE];
+#pragma unroll
+    for (int h = 0; h < HE; ++h) {
+        const int e = min(tid + h * kMuT, LP - 1), ly = e / LZ, lz = e - ly * LZ;
+        hoff[h] = (unsigned)(wrapc(y0 - H + ly, P.ny) * P.nz + wrapc(z0 - H + lz, P.nz)) * (unsigned)sizeof(TS);
+    }
+    auto fetch = [&](int x, TS (&v)[HE]) {   // past the chunk wrapped, and not used
+        x = P.nx >= 8 ? (x < 0 ? x + P.nx : (x >= P.nx ? x - P.nx : x)) : wrapc(x, P.nx);
+        const TS *r = rho + (size_t)x * pl;
+#pragma unroll
+        for (int h = 0; h < HE; ++h) v[h] = *lane_bytes(r, hoff[h]);
+    };
+    auto store = [&](int slot, const TS (&v)[HE]) {
+#pragma unroll
+        for (int h = 0; h < HE; ++h)
+            if ((h + 1) * kMuT <= LP || tid + h * kMuT < LP) s_rho[slot][tid + h * kMuT] = v[h];
+    };
+    TS va[HE], vb[HE];
+    {
+        TS v[2 * H][HE];
+#pragma unroll
+        for (int k = 0; k < 2 * H; ++k) fetch(xa - H + k, v[k]);
+#pragma unroll
+        for (int k = 0; k < 2 * H; ++k) store(k, v[k]);
+    }
+    fetch(xa + H, va);
+    fetch(xa + H + 1, vb);
+    const int base = (ty + H) * LZ + tz + H;
+    const unsigned jb = (unsigned)(inr ? y * P.nz + z : 0) * (unsigned)sizeof(TS);
+    int s0 = 0;   // ring slot of plane x - H
+    auto step = [&](int x, TS (&v)[HE]) {
+        int slot[2 * H + 1];
+#pragma unroll
+        for (int d = 0; d <= 2 * H; ++d) slot[d] = s0 + d >= R ? s0 + d - R : s0 + d;
+        store(slot[2 * H], v);   // plane x + H
+        __syncthreads();
+        fetch(x + H + 2, v);
+        if (inr) {
+            const size_t I = (size_t)x * pl;
+            const TS d = s_rho[slot[H]][base];
+            if (!solid)
+                *lane_bytes(mu + I, jb) = mu_node<TS>(P, [&](int dx, int dy, int dz) { return s_rho[slot[dx + H]][base + dy * LZ + dz]; });
+            else if (rho_solid) *lane_bytes(rho_solid + I, jb) = d;
+            if (rho_copy) *lane_bytes(rho_copy + I, jb) = d;
+        }
+        s0 = s0 + 1 == R ? 0 : s0 + 1;
+    };
+    int x = xa;
+    for (; x + 1 < xb; x += 2) {
+        step(x, va);
+        step(x + 1, vb);
+    }
+    if (x < xb) step(x, va);
+}
+
 }  // namespace
+
+// x planes per workgroup of k_mu_march, 0: k_mu_columns.  The march from 6 million nodes of
+// 4-byte densities on, where the tiles fill: us per launch, columns against march, FP32:
+// 128^3 17.7 / 18.0, 1024x64x64 23 / 24, 192^3 42 / 38, 256^3 75 / 66, 384x384x256 150 / 127,
+// 512x512x256 265 / 209 (FP16 265 / 216); tiles of one row (3001x1x501) 14 / 36.  Chunks of 32,
+// 16 or 8 planes: 256^3 73 / 66 / 70, 512x512x256 209 / 222 / 250, 384x384x256 135 / 127 / 142,
+// 192^3 45 / 42 / 38.  CPMP_MU=columns or =march (chunks of CPMP_XC, else 8) overrides.
+int mu_march_chunk(int nx, int ny, int nz, int form) {
+    if (fp64_storage(form)) return 0;
+    const long long tiles = (long long)((ny + kTileY - 1) / kTileY) * ((nz + kTileZ - 1) / kTileZ);
+    if (const char *e = std::getenv("CPMP_MU")) {
+        const char *x = std::getenv("CPMP_XC");
+        if (std::strcmp(e, "columns") == 0) return 0;
+        if (std::strcmp(e, "march") == 0) return x ? std::min(std::max(std::atoi(x), 1), 1024) : 8;
+    }
+    if ((long long)nx * ny * nz < 6000000 || 10ll * ny * nz < 7 * tiles * kTileY * kTileZ) return 0;
+    return (nx + 31) / 32 * tiles >= 8192 ? 32 : (nx + 15) / 16 * tiles >= 4096 ? 16 : 8;
+}
 
 // x planes per workgroup of k_mu_columns: enough workgroups for 8 waves per SIMD, at most 16
 // (256^3 FP32 step 525 us, with 32 planes 530)
 template <class TS>
 static hipError_t launch(cpmp_ctx *c, void *rho_copy) {
+    if constexpr (sizeof(TS) == 4) {
+        if (c->mu_chunk > 0) {
+            const int xc = c->mu_chunk, ntz = (c->p.nz + kTileZ - 1) / kTileZ, nty = (c->p.ny + kTileY - 1) / kTileY;
+            const dim3 grid((unsigned)(ntz * nty * ((c->p.nx + xc - 1) / xc)));
+            auto go = [&](auto h) {
+                hipLaunchKernelGGL((k_mu_march<TS, decltype(h)::value>), grid, dim3(kMuT), 0, c->stream, c->dp, (const TS *)c->rho,
+                                   (TS *)c->mu, (TS *)c->rho_next, (TS *)rho_copy, xc, ntz, nty);
+            };
+            if (c->dp.lap_points == 7) go(std::integral_constant<int, 3>{});
+            else go(std::integral_constant<int, 2>{});
+            return hipGetLastError();
+        }
+    }
     const int ncb = (int)blocks_for((long long)c->p.ny * c->p.nz);
     const int xc = std::max(1, std::min(16, c->p.nx * ncb / 2048));
     const dim3 grid((unsigned)(ncb * ((c->p.nx + xc - 1) / xc)));
