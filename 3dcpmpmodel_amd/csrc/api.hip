@@ -305,7 +305,7 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
         c->dp.nty = p->ny / kTileY;
         c->dp.ntz = p->nz / kTileZ;
     }
-    parts.push_back({(void **)&c->mv, 3 * (size_t)c->N * sizeof(double)});
+    parts.push_back({&c->mv, 3 * scal});
     parts.push_back({(void **)&c->mu_w, 2 * (size_t)c->NXY * sizeof(double)});
     parts.push_back({(void **)&c->red, reduce_scratch_doubles() * sizeof(double)});
     parts.push_back({(void **)&c->staging, (size_t)c->N * sizeof(double)});
@@ -322,7 +322,7 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
         hipMemsetAsync(c->rho, 0, c->N * c->scal_bytes, c->stream) != hipSuccess ||
         hipMemsetAsync(c->mu, 0, c->N * c->scal_bytes, c->stream) != hipSuccess ||
         (c->rho_next && hipMemsetAsync(c->rho_next, 0, c->N * c->scal_bytes, c->stream) != hipSuccess) ||
-        hipMemsetAsync(c->mv, 0, 3 * c->N * sizeof(double), c->stream) != hipSuccess ||
+        hipMemsetAsync(c->mv, 0, 3 * (size_t)c->N * c->scal_bytes, c->stream) != hipSuccess ||
         hipMemsetAsync(c->mu_w, 0, 2 * c->NXY * sizeof(double), c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
         return fail(CPMP_EHIP, "initial clear");
@@ -352,7 +352,7 @@ int cpmp_get_params(cpmp_ctx *c, cpmp_params *out) {
 
 int cpmp_memory(cpmp_ctx *c, int64_t *bytes) {
     if (!valid_ctx(c) || !bytes) return set_error(CPMP_EINVAL, "bad context or output");
-    *bytes = (int64_t)(2 * (size_t)c->N * 19 * c->pop_bytes + 2 * c->N * c->scal_bytes + 4 * c->N * sizeof(double)
+    *bytes = (int64_t)(2 * (size_t)c->N * 19 * c->pop_bytes + 5 * c->N * c->scal_bytes + c->N * sizeof(double)
                        + 2 * c->NXY * sizeof(double) + reduce_scratch_doubles() * sizeof(double) + c->fuse_bytes);
     return CPMP_OK;
 }
@@ -364,7 +364,7 @@ int cpmp_init_reference(cpmp_ctx *c, double radius, double width, double rg, dou
     HIPCHK(hipSetDevice(c->p.device));
     HIPCHK(launch_init_reference(c, radius, width, rg, rl, solid));
     HIPCHK(sync_reference_density(c));
-    HIPCHK(hipMemsetAsync(c->mv, 0, 3 * c->N * sizeof(double), c->stream));
+    HIPCHK(hipMemsetAsync(c->mv, 0, 3 * (size_t)c->N * c->scal_bytes, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->step = 0;
     c->mv_valid = false;
@@ -378,7 +378,7 @@ int cpmp_init_splash(cpmp_ctx *c, double radius, double width, double film_z, do
     HIPCHK(hipSetDevice(c->p.device));
     HIPCHK(launch_init_splash(c, radius, width, film_z, rg, rl));
     HIPCHK(sync_reference_density(c));
-    HIPCHK(hipMemsetAsync(c->mv, 0, 3 * c->N * sizeof(double), c->stream));
+    HIPCHK(hipMemsetAsync(c->mv, 0, 3 * (size_t)c->N * c->scal_bytes, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->step = 0;
     c->mv_valid = false;
@@ -393,7 +393,7 @@ int cpmp_init_spheres(cpmp_ctx *c, const cpmp_init_desc *d) {
     HIPCHK(hipSetDevice(c->p.device));
     HIPCHK(launch_init_spheres(c, d));
     HIPCHK(sync_reference_density(c));
-    HIPCHK(hipMemsetAsync(c->mv, 0, 3 * c->N * sizeof(double), c->stream));
+    HIPCHK(hipMemsetAsync(c->mv, 0, 3 * (size_t)c->N * c->scal_bytes, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->step = 0;
     c->mv_valid = false;
@@ -408,7 +408,7 @@ int cpmp_init_from_rho(cpmp_ctx *c, const double *rho) {
     HIPCHK(launch_scalar_from_double(c, c->staging, c->rho));
     HIPCHK(sync_reference_density(c));
     HIPCHK(launch_feq_from_rho(c));
-    HIPCHK(hipMemsetAsync(c->mv, 0, 3 * c->N * sizeof(double), c->stream));
+    HIPCHK(hipMemsetAsync(c->mv, 0, 3 * (size_t)c->N * c->scal_bytes, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->step = 0;
     c->mv_valid = false;
@@ -493,7 +493,14 @@ int cpmp_get_field(cpmp_ctx *c, int field, double *host) {
         HIPCHK(e);
     } break;
     case CPMP_FIELD_MV:
-        HIPCHK(hipMemcpyAsync(host, c->mv, 3 * nb, hipMemcpyDeviceToHost, c->stream));
+        if (c->scal_bytes == sizeof(double)) {
+            HIPCHK(hipMemcpyAsync(host, c->mv, 3 * nb, hipMemcpyDeviceToHost, c->stream));
+            break;
+        }
+        for (int k = 0; k < 3; ++k) {
+            HIPCHK(launch_scalar_to_double(c, (const char *)c->mv + (size_t)k * c->N * c->scal_bytes, c->staging));
+            HIPCHK(hipMemcpyAsync(host + (size_t)k * c->N, c->staging, nb, hipMemcpyDeviceToHost, c->stream));
+        }
         break;
     default:
         return set_error(CPMP_EINVAL, "field %d", field);

@@ -73,7 +73,7 @@ struct cpmp_ctx {
     // workspace of the adjoint, kept for the next call up to kAdjKeep bytes
     char *adj_ws = nullptr;
     size_t adj_ws_bytes = 0;
-    double *mv = nullptr;       // 3*N, MV of the last step
+    void *mv = nullptr;         // 3*N values of the scalar type, MV of the last step
     double *mu_w = nullptr;     // 2*NXY: bottom then top
     double *red = nullptr;      // reduction partials
     double *staging = nullptr;  // N doubles

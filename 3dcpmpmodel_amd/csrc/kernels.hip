@@ -188,7 +188,7 @@ __global__ void __launch_bounds__(kWallTile * kWallTile) k_wall_tile(const DevPa
 template <class TF, class TS, class TC, bool MV, bool GUO = false>
 __global__ void __launch_bounds__(TPB) k_collide(const DevParams P, const TF *__restrict__ fin, TF *__restrict__ fout,
                                                  const TS *__restrict__ rho, const TS *__restrict__ mu,
-                                                 double *__restrict__ mv, TS *__restrict__ uout,
+                                                 TS *__restrict__ mv, TS *__restrict__ uout,
                                                  const TS *__restrict__ rref) {
     const NodeIdx nd = node_from_grid(P);
     if (!nd.ok) return;
@@ -236,9 +236,9 @@ __global__ void __launch_bounds__(TPB) k_collide(const DevParams P, const TF *__
     }
     if (MV) {
         const TC h = TC(0.5) / r;
-        mv[I] = (double)(u[0] + Fx * h);
-        mv[N + I] = (double)(u[1] + Fy * h);
-        mv[2 * N + I] = (double)(u[2] + Fz * h);
+        mv[I] = (TS)(u[0] + Fx * h);
+        mv[N + I] = (TS)(u[1] + Fy * h);
+        mv[2 * N + I] = (TS)(u[2] + Fz * h);
     }
     // post-collision values stay at this node; the next step pulls them (FP16:
     // shifted by the density the puller has now, or this node's when bounced back)
@@ -388,7 +388,7 @@ __device__ __forceinline__ void ring_dest(int ly, int lz, int &dy, int &dz, int 
 template <class TF, class TS, class TC, bool MV, bool RS, bool UR, bool NW, bool QPR, bool GUO>
 __global__ void __launch_bounds__(MT) k_collide_march(const DevParams P, const TF *__restrict__ fin,
                                                        TF *__restrict__ fout, const TS *__restrict__ rho,
-                                                       const TS *__restrict__ mu, double *__restrict__ mv,
+                                                       const TS *__restrict__ mu, TS *__restrict__ mv,
                                                        TS *__restrict__ uout, int ntz, int nty,
                                                        TS *__restrict__ rho_next, TS *__restrict__ rbuf,
                                                        TS *__restrict__ cbuf, int remap, const TS *__restrict__ rref) {
@@ -638,9 +638,9 @@ __global__ void __launch_bounds__(MT) k_collide_march(const DevParams P, const T
                 }
                 if (MV) {
                     const TC h = TC(0.5) / r;
-                    mv[I] = (double)(u[0] + Fx * h);
-                    mv[N + I] = (double)(u[1] + Fy * h);
-                    mv[2 * N + I] = (double)(u[2] + Fz * h);
+                    mv[I] = (TS)(u[0] + Fx * h);
+                    mv[N + I] = (TS)(u[1] + Fy * h);
+                    mv[2 * N + I] = (TS)(u[2] + Fz * h);
                 }
             } else {
 #pragma unroll
@@ -1110,7 +1110,7 @@ __device__ __forceinline__ void block_reduce(double (&v)[RED_VALS], const int (&
 
 template <class TS>
 __global__ void __launch_bounds__(TPB) k_reduce(const DevParams P, const TS *__restrict__ rho,
-                                                const double *__restrict__ mv, int has_mv, double *__restrict__ part) {
+                                                const TS *__restrict__ mv, int has_mv, double *__restrict__ part) {
     const int kind[RED_VALS] = {0, 0, 1, 1, 2, 2, 0, 0, 0, 0, 0, 0};
     double v[RED_VALS] = {0, 0, 1e300, 1e300, -1e300, 0, 0, 0, 0, 0, 0, 0};
     const long long stride = (long long)gridDim.x * TPB;
@@ -1123,7 +1123,7 @@ __global__ void __launch_bounds__(TPB) k_reduce(const DevParams P, const TS *__r
         v[4] = fmax(v[4], d);
         v[10] += 1;
         if (has_mv) {
-            const double a = mv[I], b = mv[P.N + I], e = mv[2 * P.N + I];
+            const double a = (double)mv[I], b = (double)mv[P.N + I], e = (double)mv[2 * P.N + I];
             const double m2 = a * a + b * b + e * e;
             v[5] = fmax(v[5], m2);
             v[6] += d * a; v[7] += d * b; v[8] += d * e;
@@ -1304,7 +1304,7 @@ hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool last) {
         if (c->collide_v1) {
             auto v1 = [&](auto mv_t, auto guo_t) {
                 hipLaunchKernelGGL((k_collide<TF, TS, TC, decltype(mv_t)::value, decltype(guo_t)::value>), node_grid(c->dp),
-                                   dim3(TPB), 0, c->stream, c->dp, fin, fout, rho, mu, c->mv, uout, ref_buffer<TS>(c));
+                                   dim3(TPB), 0, c->stream, c->dp, fin, fout, rho, mu, (TS *)c->mv, uout, ref_buffer<TS>(c));
             };
             if (guo) { if (want_mv) v1(std::true_type{}, std::true_type{}); else v1(std::false_type{}, std::true_type{}); }
             else { if (want_mv) v1(std::true_type{}, std::false_type{}); else v1(std::false_type{}, std::false_type{}); }
@@ -1323,7 +1323,7 @@ hipError_t launch_collide(cpmp_ctx *c, bool want_mv, void *uout_v, bool last) {
                     hipLaunchKernelGGL((k_collide_march<TF, TS, TC, decltype(mv_t)::value, decltype(rs_t)::value,
                                                         decltype(ur_t)::value, decltype(nw_t)::value,
                                                         decltype(qp_t)::value, decltype(guo_t)::value>),
-                                       grid, dim3(MT), 0, c->stream, c->dp, fin, fout, rho, mu, c->mv, uout, ntz, nty, rn,
+                                       grid, dim3(MT), 0, c->stream, c->dp, fin, fout, rho, mu, (TS *)c->mv, uout, ntz, nty, rn,
                                        rb, cb, remap, ref_buffer<TS>(c));
                 };
                 // Guo forcing: one specialisation per (MV, RS, UR, NW), with the Qp path
@@ -1545,7 +1545,7 @@ hipError_t launch_type(cpmp_ctx *c, double *out) {
 hipError_t launch_reduce_into(cpmp_ctx *c, double *part, double *host_out) {
     hipError_t e = dispatch(c->form, [&](auto fm) {
         using TS = typename decltype(fm)::TS;
-        hipLaunchKernelGGL(k_reduce<TS>, dim3(RED_BLOCKS), dim3(TPB), 0, c->stream, c->dp, (const TS *)c->rho, c->mv,
+        hipLaunchKernelGGL(k_reduce<TS>, dim3(RED_BLOCKS), dim3(TPB), 0, c->stream, c->dp, (const TS *)c->rho, (const TS *)c->mv,
                            c->mv_valid ? 1 : 0, part);
         return hipGetLastError();
     });

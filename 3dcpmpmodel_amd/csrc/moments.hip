@@ -120,7 +120,7 @@ struct StepArgs {
     TC *eout;
     const TS *rho, *mu;
     TS *rho_out;
-    double *mv;           // u + F / (2 rho) (DIAG, may be null)
+    TS *mv;               // u + F / (2 rho) (DIAG, may be null)
     TS *uout;             // adjoint tape: u, grad mu, grad rho (DIAG, may be null)
     int ntz, nty, xc;
 };
@@ -332,9 +332,9 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 ? 4 : 2) k_moment_step
                 }
                 if (A.mv) {
                     const TC h = TC(0.5) / r;
-                    A.mv[I] = (double)(u[0] + Fx * h);
-                    A.mv[N + I] = (double)(u[1] + Fy * h);
-                    A.mv[2 * N + I] = (double)(u[2] + Fz * h);
+                    A.mv[I] = (TS)(u[0] + Fx * h);
+                    A.mv[N + I] = (TS)(u[1] + Fy * h);
+                    A.mv[2 * N + I] = (TS)(u[2] + Fz * h);
                 }
             }
         } else {
@@ -427,7 +427,7 @@ using TileRow = Tile<1, 192>;
 using TileBox = Tile<12, 32>;
 
 template <class TF, class TS, class TC>
-hipError_t launch_form(cpmp_ctx *c, bool in_p, bool out_p, double *mv, TS *uout) {
+hipError_t launch_form(cpmp_ctx *c, bool in_p, bool out_p, void *mv, TS *uout) {
     const DevParams &P = c->dp;
     StepArgs<TF, TS, TC> a;
     // moments alternate between c->mom and the population set that is not current; the
@@ -444,7 +444,7 @@ hipError_t launch_form(cpmp_ctx *c, bool in_p, bool out_p, double *mv, TS *uout)
     a.rho = (const TS *)c->rho;
     a.mu = (const TS *)c->mu;
     a.rho_out = (TS *)c->rho_next;
-    a.mv = mv;
+    a.mv = (TS *)mv;
     a.uout = uout;
     const bool nw = P.lo == 0 && P.hi == 0, diag = mv || uout;
     const int fc = P.forcing == 1 ? kGuo : P.qp_on ? kQp : kPlain;
@@ -515,7 +515,7 @@ size_t moment_bytes(int nx, int ny, int nz, int form) {
 }
 
 hipError_t launch_moment_step(cpmp_ctx *c, bool out_pops, bool want_mv, void *uout) {
-    double *mv = want_mv ? c->mv : nullptr;
+    void *mv = want_mv ? c->mv : nullptr;
     const bool in_pops = c->mom_at == 0;
     hipError_t e = hipErrorInvalidValue;
     switch (c->form) {
