@@ -26,7 +26,7 @@ Q = 19
 EXPORTS = [
     "cpmp_set_multiphase", "cpmp_default_params", "cpmp_dim_conversion", "cpmp_eos_pressure", "cpmp_eos_mu",
     "cpmp_coexistence", "cpmp_cocurve_lookup", "cpmp_create", "cpmp_destroy", "cpmp_get_params",
-    "cpmp_memory", "cpmp_init_reference", "cpmp_init_splash", "cpmp_init_spheres", "cpmp_init_from_rho",
+    "cpmp_memory", "cpmp_release_workspace", "cpmp_init_reference", "cpmp_init_splash", "cpmp_init_spheres", "cpmp_init_from_rho",
     "cpmp_set_wall_mu", "cpmp_step", "cpmp_sync", "cpmp_step_count", "cpmp_get_field",
     "cpmp_set_field", "cpmp_reduce", "cpmp_reduce_noalloc", "cpmp_contact_angle", "cpmp_cap_fit", "cpmp_probe",
     "cpmp_laplace_jump",
@@ -100,6 +100,7 @@ def _load():
     L.cpmp_destroy.argtypes = [p]
     L.cpmp_get_params.argtypes = [p, C.POINTER(Params)]
     L.cpmp_memory.argtypes = [p, C.POINTER(C.c_int64)]
+    L.cpmp_release_workspace.argtypes = [p, C.POINTER(C.c_int64)]
     L.cpmp_init_reference.argtypes = [p, d, d, d, d, d]
     L.cpmp_init_splash.argtypes = [p, d, d, d, d, d]
     L.cpmp_init_spheres.argtypes = [p, C.POINTER(InitDesc)]
@@ -336,7 +337,7 @@ class Lattice:
         """cpmp_adjoint.  tape_budget_bytes: trailing steps taped in the first
         forward run instead of recomputed (0: recompute everything, -1: half of
         the free device memory).  memory_limit_bytes: device bytes the call may
-        allocate (0: the free device memory less 2 GiB); segments whose tape does
+        use (0: the free device memory less 2 GiB); segments whose tape does
         not fit are recomputed in sub-segments."""
         nxy = self.p.nx * self.p.ny
         t = np.ascontiguousarray(target, np.float64).ravel()
@@ -392,4 +393,10 @@ class Lattice:
     def memory(self):
         b = C.c_int64()
         check(lib.cpmp_memory(self.h, C.byref(b)))
+        return b.value
+
+    def release_workspace(self):
+        """cpmp_release_workspace: the bytes returned"""
+        b = C.c_int64()
+        check(lib.cpmp_release_workspace(self.h, C.byref(b)))
         return b.value

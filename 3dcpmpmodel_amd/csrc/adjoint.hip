@@ -634,7 +634,7 @@ int make_plan(cpmp_ctx *c, const cpmp_adj_desc *d, AdjPlan &q) {
     if (need_free) {
         const hipError_t e = hipMemGetInfo(&fr, &tot);
         if (e != hipSuccess) return set_error(CPMP_EHIP, "hipMemGetInfo: %s", hipGetErrorString(e));
-        fr += c->adj_ws_bytes;   // the kept workspace is reused or returned first
+        fr += workspace_idle(c->p.device);   // reused or returned first
     }
     long long budget = d->tape_budget_bytes < 0 ? (long long)(fr / 2) : d->tape_budget_bytes;
     q.ntaped = (int)std::min<long long>(budget / (long long)q.per_tape, d->nsteps);
@@ -754,6 +754,8 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
     const size_t sb = c->scal_bytes;
     char *ckpt = nullptr, *subck = nullptr, *fin = nullptr, *tape = nullptr, *tape2 = nullptr;
     double *buf = nullptr, *tgt = nullptr;
+    char *ws = nullptr;      // the workspace, where it is one block that is kept
+    size_t ws_bytes = 0;
     bool kept = false;
     // overlapped schedule: the recompute runs on the context's state on stream s2
     hipStream_t s2 = nullptr;
@@ -771,20 +773,22 @@ extern "C" int cpmp_adjoint(cpmp_ctx *c, const cpmp_adj_desc *d, double *J, doub
         size_t need = 0;
         for (auto &w : part_of) need += padded(w.n);
         kept = need <= kAdjKeep;
-        if (c->adj_ws && (!kept || c->adj_ws_bytes < need)) {
-            (void)hipFree(c->adj_ws);
-            c->adj_ws = nullptr;
-            c->adj_ws_bytes = 0;
+        ws = workspace_take(c->p.device, &ws_bytes);
+        // a block larger than the call's limit does not stay behind it
+        const size_t most = d->memory_limit_bytes > 0 ? std::max((size_t)d->memory_limit_bytes, need) : SIZE_MAX;
+        if (ws && (!kept || ws_bytes < need || ws_bytes > most)) {
+            (void)hipFree(ws);
+            ws = nullptr;
         }
-        if (kept && !c->adj_ws) {
-            AHIP(hipMalloc((void **)&c->adj_ws, need));
-            c->adj_ws_bytes = need;
+        if (kept && !ws) {
+            AHIP(device_malloc(c->p.device, (void **)&ws, need));
+            ws_bytes = need;
         }
         size_t at = 0;
         for (auto &w : part_of) {
             if (w.n == 0) continue;
-            if (kept) *w.p = c->adj_ws + at;
-            else AHIP(hipMalloc((void **)w.p, w.n));
+            if (kept) *w.p = ws + at;
+            else AHIP(device_malloc(c->p.device, (void **)w.p, w.n));
             at += padded(w.n);
         }
         if (q.pipe) {
@@ -983,6 +987,10 @@ done:
     }
     for (hipEvent_t ev : {ev_first, ev_tape[0], ev_tape[1], ev_rev[0], ev_rev[1]})
         if (ev) (void)hipEventDestroy(ev);
+    if (ws) {
+        if (rc != CPMP_OK) (void)hipStreamSynchronize(s);
+        workspace_give(c->p.device, ws, ws_bytes);
+    }
     if (!kept)
         for (void *w : {(void *)ckpt, (void *)subck, (void *)fin, (void *)tape, (void *)tape2, (void *)buf, (void *)tgt})
             if (w) (void)hipFree(w);

@@ -11,6 +11,8 @@
 #include <cstdio>
 #include <cstring>
 #include <fstream>
+#include <map>
+#include <mutex>
 #include <sstream>
 #include <string>
 #include <vector>
@@ -27,6 +29,82 @@ int set_error(int code, const char *fmt, ...) {
     va_end(ap);
     g_err = buf;
     return code;
+}
+
+// ---------------------------------------------------------------------------
+// what the library holds of a device beside its contexts' own buffers
+namespace {
+struct DeviceShare {
+    int contexts = 0;         // open on the device
+    char *idle = nullptr;     // the adjoint workspace no call is using
+    size_t idle_bytes = 0;
+};
+std::mutex g_share_mu;
+std::map<int, DeviceShare> g_share;
+}  // namespace
+
+char *workspace_take(int device, size_t *bytes) {
+    std::lock_guard<std::mutex> lock(g_share_mu);
+    DeviceShare &s = g_share[device];
+    char *p = s.idle;
+    *bytes = s.idle_bytes;
+    s.idle = nullptr;
+    s.idle_bytes = 0;
+    return p;
+}
+
+void workspace_give(int device, char *block, size_t bytes) {
+    {
+        std::lock_guard<std::mutex> lock(g_share_mu);
+        DeviceShare &s = g_share[device];
+        if (!s.idle || s.idle_bytes < bytes) {
+            std::swap(s.idle, block);
+            std::swap(s.idle_bytes, bytes);
+        }
+    }
+    if (block) (void)hipFree(block);
+}
+
+size_t workspace_idle(int device) {
+    std::lock_guard<std::mutex> lock(g_share_mu);
+    return g_share[device].idle_bytes;
+}
+
+size_t workspace_release(int device) {
+    size_t bytes = 0;
+    char *p = workspace_take(device, &bytes);
+    if (p) (void)hipFree(p);
+    return bytes;
+}
+
+hipError_t device_malloc(int device, void **p, size_t n) {
+    hipError_t e = hipMalloc(p, n);
+    if (e != hipSuccess && workspace_release(device) > 0) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, n);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
+static void context_opened(cpmp_ctx *c) {
+    std::lock_guard<std::mutex> lock(g_share_mu);
+    c->open = true;
+    ++g_share[c->p.device].contexts;
+}
+
+// the last context of a device takes the kept workspace with it
+static void context_closed(cpmp_ctx *c) {
+    if (!c->open) return;
+    bool last;
+    {
+        std::lock_guard<std::mutex> lock(g_share_mu);
+        last = --g_share[c->p.device].contexts == 0;
+    }
+    if (last) workspace_release(c->p.device);
 }
 
 }  // namespace cpmp
@@ -312,7 +390,7 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
     auto padded = [](size_t n) { return n < ((size_t)1 << 20) ? (n + 255) / 256 * 256 : (n + 65535) / 65536 * 65536; };
     size_t total = 0;
     for (const Part &w : parts) total += padded(w.n);
-    if (hipMalloc((void **)&c->block, total) != hipSuccess) return fail(CPMP_ENOMEM, "the lattice's buffers");
+    if (device_malloc(p->device, (void **)&c->block, total) != hipSuccess) return fail(CPMP_ENOMEM, "the lattice's buffers");
     size_t at = 0;
     for (const Part &w : parts) {
         *w.p = c->block + at;
@@ -326,6 +404,7 @@ int cpmp_create(const cpmp_params *p, cpmp_ctx **out) {
         hipMemsetAsync(c->mu_w, 0, 2 * c->NXY * sizeof(double), c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
         return fail(CPMP_EHIP, "initial clear");
+    context_opened(c);
     *out = c;
     return CPMP_OK;
 }
@@ -334,7 +413,7 @@ int cpmp_destroy(cpmp_ctx *c) {
     if (!c) return CPMP_OK;
     if (c->stream) { hipSetDevice(c->p.device); hipStreamSynchronize(c->stream); }
     if (c->block) hipFree(c->block);
-    if (c->adj_ws) hipFree(c->adj_ws);
+    context_closed(c);
     if (c->timers) {
         for (auto &e : c->timers->ev) if (e) hipEventDestroy(e);
         delete c->timers;
@@ -354,6 +433,14 @@ int cpmp_memory(cpmp_ctx *c, int64_t *bytes) {
     if (!valid_ctx(c) || !bytes) return set_error(CPMP_EINVAL, "bad context or output");
     *bytes = (int64_t)(2 * (size_t)c->N * 19 * c->pop_bytes + 5 * c->N * c->scal_bytes + c->N * sizeof(double)
                        + 2 * c->NXY * sizeof(double) + reduce_scratch_doubles() * sizeof(double) + c->fuse_bytes);
+    return CPMP_OK;
+}
+
+int cpmp_release_workspace(cpmp_ctx *c, int64_t *bytes) {
+    if (!valid_ctx(c)) return set_error(CPMP_EINVAL, "bad context");
+    HIPCHK(hipSetDevice(c->p.device));
+    const size_t n = workspace_release(c->p.device);
+    if (bytes) *bytes = (int64_t)n;
     return CPMP_OK;
 }
 
@@ -478,7 +565,7 @@ int cpmp_get_field(cpmp_ctx *c, int field, double *host) {
     case CPMP_FIELD_VEL:
     case CPMP_FIELD_FORCE: {
         double *tmp = nullptr;
-        HIPCHK(hipMalloc((void **)&tmp, 3 * nb));
+        HIPCHK(device_malloc(c->p.device, (void **)&tmp, 3 * nb));
         hipError_t e;
         if (field == CPMP_FIELD_VEL) {
             e = launch_velocity(c, tmp);

@@ -54,7 +54,8 @@ struct cpmp_ctx {
     size_t pop_bytes = 0;       // bytes of one population value
     size_t scal_bytes = 0;      // bytes of one rho/mu value
     hipStream_t stream = nullptr;
-    char *block = nullptr;      // the allocation that holds every buffer below but adj_ws
+    char *block = nullptr;      // the allocation that holds every buffer below
+    bool open = false;          // counted among the device's contexts
     void *f[2] = {nullptr, nullptr};
     int cur = 0;
     void *rho = nullptr, *mu = nullptr;
@@ -70,9 +71,6 @@ struct cpmp_ctx {
     void *mom = nullptr;
     int mom_at = 0;
     size_t fuse_bytes = 0;
-    // workspace of the adjoint, kept for the next call up to kAdjKeep bytes
-    char *adj_ws = nullptr;
-    size_t adj_ws_bytes = 0;
     void *mv = nullptr;         // 3*N values of the scalar type, MV of the last step
     double *mu_w = nullptr;     // 2*NXY: bottom then top
     double *red = nullptr;      // reduction partials
@@ -122,10 +120,23 @@ size_t moment_bytes(int nx, int ny, int nz, int form);
 // the populations, to moments and (out_pops) populations; rho_next receives the new
 // density of the fluid nodes
 hipError_t launch_moment_step(cpmp_ctx *c, bool out_pops, bool want_mv, void *uout);
-// Adjoint workspaces up to this size stay with the context: allocating and freeing them
+// Adjoint workspaces up to this size are kept for the next call: allocating and freeing them
 // took 3 to 50 ms a call, more than the sweep of a small lattice (128x128x64 FP32, 40 taped
-// steps: 54 ms a call, 13.7 ms of it work); larger ones are returned after the call.
+// steps: 54 ms a call, 13.7 ms of it work); larger ones are returned after the call.  Each
+// device keeps at most one idle block, which any of its contexts' calls takes for itself
+// while it runs; it is returned when the device's last context closes, when an allocation of
+// the library finds too little memory, and by cpmp_release_workspace.
 constexpr size_t kAdjKeep = (size_t)8 << 30;
+// the device's idle block, from now on the caller's (null: none)
+char *workspace_take(int device, size_t *bytes);
+// gives a block back that no work uses any more; the larger of it and an idle one is kept
+void workspace_give(int device, char *block, size_t bytes);
+size_t workspace_idle(int device);
+// frees the idle block; its bytes
+size_t workspace_release(int device);
+// hipMalloc on the current device, which `device` names; once more without the idle block if
+// memory is short.  A failure leaves no error behind for a later hipGetLastError.
+hipError_t device_malloc(int device, void **p, size_t n);
 constexpr int kTileY = 8, kTileZ = 32;   // in-plane tile of the march kernels and of tiled population storage
 constexpr int kWallTile = 16;             // columns per edge of the wall-fill tiles (16 x 16 workgroups)
 // copy one population set between the device layout and the reference node order

@@ -125,8 +125,8 @@ typedef struct {
        recompute for every step but those of the last segment, which the working tape
        holds during the first run; < 0: half of the free device memory. */
     int64_t tape_budget_bytes;
-    /* Limit on the device bytes the call allocates (0: the free device memory less
-       2 GiB).  A segment whose tape does not fit is recomputed in sub-segments:
+    /* Limit on the device bytes the call uses, and on what it leaves kept for the next
+       (cpmp_release_workspace) (0: the free device memory less 2 GiB).  A segment whose tape does not fit is recomputed in sub-segments:
        a first pass stores sub-checkpoints, then each sub-segment is taped in turn
        (each of its steps is recomputed twice).  The result does not depend on the
        schedule. */
@@ -135,7 +135,8 @@ typedef struct {
 
 /* The schedule and memory of one adjoint call (cpmp_adjoint_plan). */
 typedef struct {
-    int64_t device_bytes;      /* device memory the call allocates besides the context */
+    int64_t device_bytes;      /* device memory the call uses besides the context, a kept
+                                  workspace (cpmp_release_workspace) included */
     int taped_steps;           /* trailing steps taped during the first forward run */
     int segments;              /* checkpoint segments before them */
     int sub_length;            /* steps per taped sub-segment (= segment length when it fits) */
@@ -176,8 +177,15 @@ int cpmp_cocurve_lookup(const char *path, double Tr, double *rhog_reduced, doubl
 int cpmp_create(const cpmp_params *p, cpmp_ctx **out);
 int cpmp_destroy(cpmp_ctx *ctx);
 int cpmp_get_params(cpmp_ctx *ctx, cpmp_params *out);
-/* device memory of the context in bytes */
+/* device memory of the context in bytes (without the adjoint's workspace) */
 int cpmp_memory(cpmp_ctx *ctx, int64_t *bytes);
+/* Device memory that cpmp_adjoint works in, up to 8 GiB, stays allocated after the call for
+   the next one on the same device, of this or another context; at most one such block per
+   device.  It is returned when the device's last context is destroyed, when an allocation of
+   the library finds too little memory, and by this call (no counterpart in the reference),
+   for callers that need the memory for allocations of their own.  bytes (may be NULL):
+   what was returned, 0 if nothing was kept. */
+int cpmp_release_workspace(cpmp_ctx *ctx, int64_t *bytes);
 
 /* ---- initial conditions (SetFlowField, FluidCuda.cu:199-241) ---- */
 /* CONTACTANGLE branch: sphere of `radius` centred at (DX/2, DY/2, radius+2), tanh
