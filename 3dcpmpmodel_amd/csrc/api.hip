@@ -119,6 +119,8 @@ using namespace cpmp;
 
 namespace {
 
+const void *mv_component(const cpmp_ctx *c, int k) { return (const char *)c->mv + (size_t)k * c->N * c->scal_bytes; }
+
 bool valid_ctx(cpmp_ctx *c) { return c != nullptr && c->stream != nullptr; }
 
 // FP16 form: after an initial state is written, its density is also the
@@ -584,9 +586,15 @@ int cpmp_get_field(cpmp_ctx *c, int field, double *host) {
             HIPCHK(hipMemcpyAsync(host, c->mv, 3 * nb, hipMemcpyDeviceToHost, c->stream));
             break;
         }
-        for (int k = 0; k < 3; ++k) {
-            HIPCHK(launch_scalar_to_double(c, (const char *)c->mv + (size_t)k * c->N * c->scal_bytes, c->staging));
-            HIPCHK(hipMemcpyAsync(host + (size_t)k * c->N, c->staging, nb, hipMemcpyDeviceToHost, c->stream));
+        if (c->collide_v1) {   // leaves the solid nodes' slots of a population set as they are
+            for (int k = 0; k < 3; ++k) {
+                HIPCHK(launch_scalar_to_double(c, mv_component(c, k), c->staging));
+                HIPCHK(hipMemcpyAsync(host + (size_t)k * c->N, c->staging, nb, hipMemcpyDeviceToHost, c->stream));
+            }
+        } else {   // one copy (each takes 15 us and more) from the buffer that holds neither populations nor moments
+            double *wide = (double *)(c->mom_at == 2 ? c->mom : c->f[c->cur ^ 1]);   // 38 bytes per node or more
+            for (int k = 0; k < 3; ++k) HIPCHK(launch_scalar_to_double(c, mv_component(c, k), wide + (size_t)k * c->N));
+            HIPCHK(hipMemcpyAsync(host, wide, 3 * nb, hipMemcpyDeviceToHost, c->stream));
         }
         break;
     default:

@@ -156,3 +156,60 @@ def test_thin_lattices_take_the_faster_path(cpmp, monkeypatch, form, dims, momen
     monkeypatch.delenv("CPMP_FUSE", raising=False)
     monkeypatch.delenv("CPMP_XC", raising=False)
     assert (memory(None) - memory("v1") >= 12 * word * n) == moments
+
+
+# what a program does between calls: it must leave the moments usable or give them up
+BETWEEN = {
+    "checkpoint": lambda g, tmp: g.checkpoint_save(str(tmp / "c.ckp")),
+    "plt": lambda g, tmp: g.write_plt(str(tmp / "c.plt")),
+    "fields": lambda g, tmp: [g.get(k) for k in ("rho", "mu", "mv", "vel", "force", "f", "type")],
+    "reduce": lambda g, tmp: g.reduce(),
+    "set": lambda g, tmp: [g.set(k, g.get(k)) for k in ("f", "rho", "mu")],
+    "reload": lambda g, tmp: (g.checkpoint_save(str(tmp / "r.ckp")), g.checkpoint_load(str(tmp / "r.ckp"))),
+}
+SETTLED = [((64, 16, 64), 4, 3, {}), ((64, 16, 64), 4, 0, {}), ((12, 13, 34), 5, 3, {}), ((20, 1, 191), 6, 3, {})]
+
+
+@pytest.mark.parametrize("form", ["fp64", "fp32", "fp32a"])
+@pytest.mark.parametrize("case", SETTLED, ids=lambda c: "x".join(map(str, c[0])) + "w%d" % c[2])
+@pytest.mark.parametrize("what", list(BETWEEN))
+def test_calls_between_runs_leave_the_run_as_it_is(cpmp, monkeypatch, tmp_path, what, case, form):
+    """after one and after two steps, when the moments sit in their own buffer and in the
+    population set that is not current: the same call between two runs of steps, against an
+    undisturbed run, bit for bit, on tiled and other lattices; and the fields it returns
+    come out the same twice"""
+    a = lattice(cpmp, monkeypatch, case, form, "moments")
+    b = lattice(cpmp, monkeypatch, case, form, "moments")
+    for n in (1, 2, 3):
+        for g in (a, b):
+            g.step(n)
+        BETWEEN[what](a, tmp_path)
+        mv = a.get("mv")
+        assert np.array_equal(mv, a.get("mv"))
+        if what != "reload":        # a checkpoint does not hold MV
+            assert np.array_equal(mv, b.get("mv"))
+    for g in (a, b):
+        g.step(2)
+    for field in ("rho", "mu", "f", "mv"):
+        assert np.array_equal(a.get(field), b.get(field)), field
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("form", ["fp64", "fp32", "fp32a"])
+def test_populations_set_between_runs_are_taken(cpmp, monkeypatch, form):
+    """the state of another lattice set over moments that are current"""
+    case = SETTLED[0]
+    for n in (1, 2):
+        a = lattice(cpmp, monkeypatch, case, form, "moments")
+        b = lattice(cpmp, monkeypatch, case, form, "moments")
+        a.step(n)
+        b.step(5)
+        for field in ("f", "rho"):
+            a.set(field, b.get(field))
+        a.step(3)
+        b.step(3)
+        for field in ("rho", "f"):
+            assert np.array_equal(a.get(field), b.get(field)), field
+        a.close()
+        b.close()
