@@ -123,11 +123,16 @@ __device__ __forceinline__ double recip64(double x) {
     return fma(fma(-x, r, 1.0), r, r);
 }
 
-// FP64 natural logarithm within 1 ulp.  x = 2^k m with m in [sqrt(1/2), sqrt(2)),
-// f = m - 1 (exact), s = f / (2 + f):  ln m = 2 atanh(s) = 2 s + s R,
-// R = 2 s^2 (1/3 + s^2/5 + s^4/7 + ..), |s| <= 0.172, so the series to s^20 / 23 leaves
-// 3e-18; written as f - (f^2/2 - s (f^2/2 + R)), where only small terms carry the rounding
-// of s.  The device library's log costs about twice the instructions.
+// FP64 natural logarithm within 0.6 ulp.  x = 2^k m with m in [sqrt(1/2), sqrt(2)),
+// f = m - 1 (exact), ln m = 2 atanh(t) = 2 t + 2 t (t^2/3 + t^4/5 + ..) with t = f / (2 + f),
+// |t| <= 0.172, so the series to t^20 / 21 leaves 6e-19 of ln m.  s is t rounded; what it leaves is
+// e / (2 + f) with e = f - s (2 + f), formed exactly by two fused steps from the rounded
+// denominator and its own error.  k ln 2 + 2 s is summed with its rounding error kept, and
+// everything small joins at the end, so one rounding decides.  k ln 2 in two parts: the
+// high one has 40 significant bits, so its product with k is exact.
+// The device library's log costs about twice the instructions.  TIGHT = false leaves the
+// two corrections out, within 3 ulp, for results that are rounded to FP32.
+template <bool TIGHT = true>
 __device__ __forceinline__ double ln64(double x) {
     if (!__builtin_amdgcn_class(x, 0x180))   // not positive, finite and non-zero
         return x == 0.0 ? -__builtin_inf() : x > 0.0 ? x : __builtin_nan("");
@@ -136,9 +141,8 @@ __device__ __forceinline__ double ln64(double x) {
     const bool low = m < 0.70710678118654752440;
     m = low ? 2.0 * m : m;
     k = low ? k - 1 : k;
-    const double f = m - 1.0, den = 2.0 + f, s = f * recip64(den), z = s * s;
-    double r = 2.0 / 23;
-    r = fma(r, z, 2.0 / 21);
+    const double f = m - 1.0, den = 2.0 + f, rd = recip64(den), s = f * rd, z = s * s;
+    double r = 2.0 / 21;
     r = fma(r, z, 2.0 / 19);
     r = fma(r, z, 2.0 / 17);
     r = fma(r, z, 2.0 / 15);
@@ -148,11 +152,12 @@ __device__ __forceinline__ double ln64(double x) {
     r = fma(r, z, 2.0 / 7);
     r = fma(r, z, 2.0 / 5);
     r = fma(r, z, 2.0 / 3);
-    r *= z;
-    const double h = 0.5 * f * f, kd = (double)k;
-    // k ln 2 in two parts: the high one has 32 significant bits, so its product is exact
-    const double hi = 0x1.62e42fee00000p-1, lo = 0x1.a39ef35793c76p-33;
-    return kd * hi - ((h - fma(s, h + r, kd * lo)) - f);
+    const double kd = (double)k, hi = 0x1.62e42fefa2000p-1, lo = 0x1.9ef35793c7673p-41, s2 = s + s;
+    if constexpr (!TIGHT) return fma(kd, hi, s2 + fma(s * z, r, kd * lo));
+    const double e = fma(-s, f - (den - 2.0), fma(-s, den, f));
+    const double big = kd * hi, t = big + s2;
+    const double lost = s2 - (t - big);   // exact: |big| > |s2| or big = 0
+    return t + (lost + fma(s * z, r, fma(kd, lo, e * (rd + rd))));
 }
 
 __device__ __forceinline__ double wave_sum(double v) {

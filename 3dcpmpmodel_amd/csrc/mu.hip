@@ -43,26 +43,29 @@ __device__ __forceinline__ float mu_eos_fast(int eos, int form, float A, float B
 // mu_eos in FP64 with ln64 and one reciprocal for all the quotients of an EOS (the closed
 // forms of mu_eos_t; for Peng-Robinson (sqrt2 - 1 + bd)(sqrt2 + 1 - bd) = 1 + 2 bd - bd^2,
 // so the quotient in its second logarithm is (sqrt2 - 1 + bd)^2 over the same denominator)
+// TIGHT: ln64's
+template <bool TIGHT>
 __device__ __forceinline__ double mu_eos_fast(const DevParams &P, double d) {
+    auto ln = [](double x) { return ln64<TIGHT>(x); };
     if (d > 9.7) d = 9.7 + (d - 9.7) * recip64(1.0 + (d - 9.7) * 1.5);   // clamp_rho
     const double A = P.A, T = P.T, bd = P.B * d, om = 1.0 - bd;
     if (P.mu_form == 1 || P.eos == EOS_PRW || P.eos == EOS_PRM) {
         const double q = 1.0 + 2.0 * bd - bd * bd, u = kSqrt2 - 1.0 + bd, r = recip64(om * q), rom = r * q, rq = r * om;
-        return T * ln64(d * rom) - P.AoPr * ln64(u * u * rq) + T * rom - A * d * rq;
+        return T * ln(d * rom) - P.AoPr * ln(u * u * rq) + T * rom - A * d * rq;
     }
     if (P.eos == EOS_RKE || P.eos == EOS_RKS) {
         const double op = 1.0 + bd, r = recip64(om * op), rom = r * op;
-        return T * ln64(d * rom) + T * rom - P.AoB * ln64(op) - A * d * (r * om);
+        return T * ln(d * rom) + T * rom - P.AoB * ln(op) - A * d * (r * om);
     }
     const double rom = recip64(om);
-    if (P.eos == EOS_VDW) return T * ln64(d * rom) + T * rom - 2.0 * A * d;
-    return T * (ln64(d) + (8.0 * bd - 9.0 * bd * bd + 3.0 * bd * bd * bd) * (rom * rom * rom)) - 2.0 * A * d;
+    if (P.eos == EOS_VDW) return T * ln(d * rom) + T * rom - 2.0 * A * d;
+    return T * (ln(d) + (8.0 * bd - 9.0 * bd * bd + 3.0 * bd * bd * bd) * (rom * rom * rom)) - 2.0 * A * d;
 }
 
 // FP32 mu of an interface node from its FP32 Laplacian term Ka * lap: the EOS part
 // in FP64, rounded once
 __device__ __forceinline__ float mu_band(const DevParams &P, float d, float kal) {
-    return (float)(P.K2s * mu_eos_fast(P, (double)d) - (double)kal);
+    return (float)(P.K2s * mu_eos_fast<false>(P, (double)d) - (double)kal);
 }
 __device__ __forceinline__ bool in_band(const DevParams &P, float d) { return d > P.band_lo && d < P.band_hi; }
 
@@ -87,7 +90,7 @@ __device__ __forceinline__ TS mu_node(const DevParams &P, Get get) {
             };
             kal = P.Ka * ((-d * 90 + ax(1, 0, 0) + ax(0, 1, 0) + ax(0, 0, 1)) / 12);
         }
-        return P.K2s * mu_eos_fast(P, d) - kal;
+        return P.K2s * mu_eos_fast<true>(P, d) - kal;
     } else {
         const float d = get(0, 0, 0);
         auto df = [&](int dx, int dy, int dz) { return (float)get(dx, dy, dz) - d; };
