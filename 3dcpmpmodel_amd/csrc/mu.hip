@@ -49,17 +49,19 @@ __device__ __forceinline__ double mu_eos_fast(const DevParams &P, double d) {
     auto ln = [](double x) { return ln64<TIGHT>(x); };
     if (d > 9.7) d = 9.7 + (d - 9.7) * recip64(1.0 + (d - 9.7) * 1.5);   // clamp_rho
     const double A = P.A, T = P.T, bd = P.B * d, om = 1.0 - bd;
+    double mu;
     if (P.mu_form == 1 || P.eos == EOS_PRW || P.eos == EOS_PRM) {
         const double q = 1.0 + 2.0 * bd - bd * bd, u = kSqrt2 - 1.0 + bd, r = recip64(om * q), rom = r * q, rq = r * om;
-        return T * ln(d * rom) - P.AoPr * ln(u * u * rq) + T * rom - A * d * rq;
-    }
-    if (P.eos == EOS_RKE || P.eos == EOS_RKS) {
+        mu = T * ln(d * rom) - P.AoPr * ln(u * u * rq) + T * rom - A * d * rq;
+    } else if (P.eos == EOS_RKE || P.eos == EOS_RKS) {
         const double op = 1.0 + bd, r = recip64(om * op), rom = r * op;
-        return T * ln(d * rom) + T * rom - P.AoB * ln(op) - A * d * (r * om);
+        mu = T * ln(d * rom) + T * rom - P.AoB * ln(op) - A * d * (r * om);
+    } else {
+        const double rom = recip64(om);
+        mu = P.eos == EOS_VDW ? T * ln(d * rom) + T * rom - 2.0 * A * d
+                              : T * (ln(d) + (8.0 * bd - 9.0 * bd * bd + 3.0 * bd * bd * bd) * (rom * rom * rom)) - 2.0 * A * d;
     }
-    const double rom = recip64(om);
-    if (P.eos == EOS_VDW) return T * ln(d * rom) + T * rom - 2.0 * A * d;
-    return T * (ln(d) + (8.0 * bd - 9.0 * bd * bd + 3.0 * bd * bd * bd) * (rom * rom * rom)) - 2.0 * A * d;
+    return om == 0.0 ? T * __builtin_inf() : mu;   // at the densest packing, where recip64 has no value
 }
 
 // FP32 mu of an interface node from its FP32 Laplacian term Ka * lap: the EOS part

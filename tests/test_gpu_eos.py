@@ -80,3 +80,16 @@ def test_every_eos(cpmp, eos, tr):
     ratio = float(np.max(np.abs(mu - ref) / bound))
     print(f"[eos] {eos}: {ratio:.3f} of the bound", flush=True)
     assert ratio < 1
+
+
+@pytest.mark.parametrize("eos", [e for e, _ in EOS_TRS])
+def test_limits(cpmp, eos):
+    """the densest packing, b d = 1, an empty node, and densities far past the clamp keep the
+    values of the closed forms"""
+    rho = np.full(N, 4.0)
+    assert np.all(device_mu(cpmp, rho, eos, 1.0, 0.25, 1.0) == np.inf)
+    rho[:] = 0.0
+    assert np.all(device_mu(cpmp, rho, eos, 1.0, 0.0625, 1.0) == -np.inf)
+    rho[:] = 1e300
+    ref, _ = mu_extended(eos, 1.0, 0.0625, 1.0, 1e300)
+    assert np.all(np.abs(device_mu(cpmp, rho, eos, 1.0, 0.0625, 1.0) - np.float64(ref)) < 1e-13)
