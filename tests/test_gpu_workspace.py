@@ -1,6 +1,7 @@
 """The adjoint's workspace between calls: reused by every context of the device, never larger
 than a call's limit, returned on request, with the last context, and to an allocation that
 would fail without it; the results do not depend on what block a call runs in."""
+import gc
 import threading
 
 import numpy as np
@@ -20,7 +21,12 @@ def used_since(free0):
 
 
 @pytest.fixture
-def free0():
+def free0(cpmp):
+    """free device memory with no workspace kept from before"""
+    gc.collect()
+    g = cpmp.Lattice(cpmp.make_params(8, 8, 8, nwall=0))
+    g.release_workspace()
+    g.close()
     torch.cuda.empty_cache()
     return torch.cuda.mem_get_info()[0]
 
