@@ -39,17 +39,16 @@ def test_interface_chemical_potential_in_fp64(cpmp, monkeypatch, form, geom):
     """The FP32 storage forms evaluate the EOS part of mu in FP64 at interface nodes
     (density inside the Maxwell gas-liquid gap less 2 % at each end) and round once:
     there mu matches the FP64 form's mu of the same (FP32) density field to 1.5 FP32
-    ulp, both for the chemical-potential march that starts a run and for the one
-    that completes the previous step's summed density (the second step of a run on a
-    periodic tiled lattice).  The walled lattice has partial tiles (13 x 36 in y, z)
+    ulp, in the first step of a run and in the second, whose densities the first
+    summed; by columns, and (periodic-long) by the march over tiles that large lattices
+    take, in chunks of 32 planes.  The walled lattice has partial tiles (13 x 36 in y, z)
     and 3 + 3 wall layers; nodes whose Laplacian reaches the wall (within 2 layers)
-    are left out there, since the wall values are stored in FP32.  periodic-long:
-    chunks of 32 planes, where many waves hold more interface nodes than they finish
-    themselves and pass the rest to the overflow kernel."""
+    are left out there, since the wall values are stored in FP32."""
     if geom.startswith("periodic"):
         dims, eos, tr, nwall, sphere = (64, 32, 64), "RKE", 0.6, 0, (32, 16, 32, 14)
-        # the fused path with the folded completion
+        # the density summed inside the collide
         monkeypatch.setenv("CPMP_XC", "32" if geom == "periodic-long" else "2")
+        monkeypatch.setenv("CPMP_MU", "march" if geom == "periodic-long" else "columns")
     else:
         dims, eos, tr, nwall, sphere = (40, 13, 36), "PRW", 0.7, 3, (20, 6, 2.5, 10)
     A, B, Tc, Rc = cpmp.set_multiphase(eos, tr)

@@ -1,13 +1,12 @@
-"""The march configuration that large lattices run, against the oracle.
+"""The configurations that large lattices run, against the oracle.
 
-Lattices of 256^3 and 512x512x256 select x-march workgroups of 32 planes in every
-storage form, 128x128x96 and similar lattices 4.  Here lattices with nx >= 64 run
-with chunks of 4, 8, 16 and 32 planes (CPMP_XC), so the 8-slot LDS ring rotates
-over long chunks, the chemical-potential march alternates its two register sets
-over many planes and the chunk-end partial planes of the summed density are
-exercised, in the FP64 form (<= 1e-10 relative on rho after 200 steps), the FP32
-form with the fused density and the completion folded into the next
-chemical-potential kernel, and the FP16 form; then every EOS in the FP32 form
+Lattices of 256^3 and 512x512x256 select x-march workgroups of 32 planes, 128x128x96
+and similar lattices 4: the population march in the FP16 form and with rates other than
+the reference's, the step on moments otherwise.  Here lattices with nx >= 64 run with
+chunks of 4 to 64 planes (CPMP_XC), so the LDS rings rotate over long chunks and the
+chunk-end partial planes of the summed density are exercised: the population march in
+the FP64 form (<= 1e-10 relative on rho after 200 steps), the FP32 and FP32A forms and
+the FP16 form, and the step on moments; then every EOS in the FP32 form
 (including the FP32 bulk chemical potential), and the large van der Waals
 striped-wall wetting configuration at a size the oracle covers, with its
 adjoint."""
@@ -32,7 +31,7 @@ GEOMS = {
     "walled": dict(dims=(64, 16, 64), eos="PRW", tr=0.70, nwall=3, init="reference", radius=13, width=5,
                    mu_w=-0.02, steps=200),
     # the periodic case with the 7-point Laplacian (PTCALCSEVENPOINT, Common.h:243-246):
-    # halo of 3 in the chemical-potential march and in the folded completion
+    # halo of 3 in the chemical potential
     "periodic7": dict(dims=(64, 16, 64), eos="RKE", tr=0.60, nwall=0, init="spheres",
                       spheres=[(20, 8, 31.5, 10), (43, 8, 33, 10)], width=5, noise=1e-4, seed=3, steps=200,
                       lap_points=7),
@@ -122,9 +121,8 @@ def test_fp64_march_long_chunks_match_oracle(cpmp, name, xc):
 @pytest.mark.parametrize("form,tol", [("fp32", 2e-4), ("fp16", 2e-2), ("fp32a", 2e-4)])
 @pytest.mark.parametrize("name", list(GEOMS))
 def test_reduced_forms_long_chunks_match_oracle(cpmp, name, form, tol, xc):
-    """fused density with chunks of 4 and 32 planes (periodic FP32: the completion
-    folded into the next step's chemical-potential kernel) against the FP64 oracle;
-    the FP32-arithmetic form (FP64 storage) forced onto the march collide, which
+    """the population march with the density summed inside it, chunks of 4 and 32 planes,
+    against the FP64 oracle; the FP32-arithmetic form (FP64 storage) forced onto the march collide, which
     these lattices would otherwise run one thread per node as the FP64 form does"""
     case = GEOMS[name]
     print(f"[production] {form} {name} xc={xc} steps={case['steps']}", flush=True)
@@ -158,22 +156,25 @@ def test_reduced_forms_long_chunks_match_oracle(cpmp, name, form, tol, xc):
     short.close()
 
 
-@pytest.mark.parametrize("name", ["periodic", "periodic7"])
-def test_folded_completion_long_chunks_is_bitwise_the_same(cpmp, name):
-    """periodic FP32 with chunks of 32 (5- and 7-point Laplacian): the completion
-    folded into the next mu kernel leaves the same bits as the completion pass
-    after every step"""
-    print(f"[production] folded completion {name}", flush=True)
-    a = device(name, cpmp, "fp32", CPMP_XC=32)
-    b = device(name, cpmp, "fp32", CPMP_XC=32)
-    for n in (1, 4, 9):
-        with env(CPMP_DEFER=0):
-            b.step(n)
-        a.step(n)
-        for field in ("rho", "mu", "f"):
-            assert np.array_equal(a.get(field), b.get(field)), (n, field)
-    a.close()
-    b.close()
+@pytest.mark.parametrize("xc", [8, 32, 64])
+@pytest.mark.parametrize("form,tol", [("fp64", TOL64), ("fp32", 2e-4), ("fp32a", 2e-4)])
+@pytest.mark.parametrize("name", list(GEOMS))
+def test_moment_runs_long_chunks_match_oracle(cpmp, name, form, tol, xc):
+    """the step on moments, which large lattices take at the reference's rates, with chunks
+    of 8 planes, of 32, and of the whole lattice"""
+    case = GEOMS[name]
+    rho0, rho_o, f_o, fluid = oracle_run(name)
+    g = device(name, cpmp, form, CPMP_COLLIDE="moments", CPMP_XC=xc)
+    for n in (1, 2, case["steps"] - 3):
+        g.step(n)
+    r = g.get("rho")[fluid]
+    err = gc.rel_err(r, rho_o[fluid]) if form == "fp64" else np.max(np.abs(r - rho_o[fluid])) / np.max(rho_o[fluid])
+    print(f"[production] moments {form} {name} xc={xc}: rho err {err:.3e}", flush=True)
+    assert err < tol
+    if form == "fp64":
+        fo, fg = f_o.reshape(19, -1), g.get("f").reshape(19, -1)
+        assert np.max(np.abs(fg[:, fluid] - fo[:, fluid])) < TOL64 * np.max(np.abs(fo[:, fluid]))
+    g.close()
 
 
 # ---------------------------------------------------------------------------
