@@ -115,6 +115,17 @@ __device__ __forceinline__ unsigned in_loop(unsigned v) {
     return v;
 }
 
+// Element i of a plane at such a base, for use in a loop.
+template <class T>
+__device__ __forceinline__ T *lane_at(T *base, unsigned i) {
+    return lane_bytes(base, in_loop(i) * (unsigned)sizeof(T));
+}
+
+// relaxation rates in the arithmetic precision, read from the kernel argument
+template <class TC> __device__ __forceinline__ const TC *rates(const DevParams &P);
+template <> __device__ __forceinline__ const double *rates<double>(const DevParams &P) { return P.ts; }
+template <> __device__ __forceinline__ const float *rates<float>(const DevParams &P) { return P.tsf; }
+
 // FP64 reciprocal: the hardware estimate and two Newton steps (within 1 ulp; finite
 // non-zero x)
 __device__ __forceinline__ double recip64(double x) {

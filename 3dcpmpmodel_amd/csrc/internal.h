@@ -59,8 +59,9 @@ struct cpmp_ctx {
     void *f[2] = {nullptr, nullptr};
     int cur = 0;
     void *rho = nullptr, *mu = nullptr;
-    // FP32 storage forms on exactly tiled lattices: density summed by the collide
-    // kernel into rho_next, tile rings and chunk partial planes for the fix-up pass
+    // rho_next: the density after the step, on lattices on moments and where the march sums
+    // it; the FP16 form's previous density.  rbuf, cbuf: tile rings and chunk partial planes
+    // of the march on exactly tiled lattices
     void *rho_next = nullptr, *rbuf = nullptr, *cbuf = nullptr;
     bool collide_v1 = false;    // one-thread-per-node collide (node_collide)
     bool moments = false;       // runs of steps carry 13 moments per node (moment_path)

@@ -41,10 +41,6 @@ hipError_t dispatch(int form, Fn &&fn) {
     return hipErrorInvalidValue;
 }
 
-// relaxation rates in the arithmetic precision, read from the kernel argument
-template <class TC> __device__ __forceinline__ const TC *rates(const DevParams &P);
-template <> __device__ __forceinline__ const double *rates<double>(const DevParams &P) { return P.ts; }
-template <> __device__ __forceinline__ const float *rates<float>(const DevParams &P) { return P.tsf; }
 
 // FP16 storage holds f_q - w_q rho_ref with rho_ref the density of the node that
 // pulls the value, in the step that wrote it (the density the collide kernel read
@@ -133,8 +129,8 @@ __global__ void __launch_bounds__(TPB) k_wall(const DevParams P, TS *__restrict_
 }
 
 // The same fill in one launch for walls of at most R (<= 4) layers (any depth with the
-// simple scheme, which reads the first fluid layer only).  With the layered scheme layer lo-d is A^d applied to the first fluid layer, A the diagonal
-// average above, so a 16 x 16 tile of columns needs the fluid layer on the tile
+// simple scheme, which reads the first fluid layer only).  With the layered scheme layer
+// lo-d is A^d applied to the first fluid layer, A the diagonal average above, so a 16 x 16 tile of columns needs the fluid layer on the tile
 // plus a halo of R columns.  The workgroup stages that patch in LDS and recomputes
 // the layers on shrinking patches with the same arithmetic (including the rounding
 // to the storage type) as the pass kernels, so the results are identical.
@@ -1174,9 +1170,9 @@ hipError_t launch_wall(cpmp_ctx *c) {
     });
 }
 
-// FP32 storage forms with the march collide sum the density inside the collide
-// kernel when the tiles cover the lattice exactly (a context created with
-// CPMP_FUSE=0 in the environment keeps the separate density pass)
+// The population march sums the density inside the collide kernel when the tiles
+// cover the lattice exactly (a context created with CPMP_FUSE=0 in the environment
+// keeps the separate density pass)
 bool fuse_geometry(int nx, int ny, int nz, int xc, size_t *ring_elems, size_t *chunk_elems) {
     if (xc < 2 || xc > MXC || nx % xc || ny % MTY || nz % MTZ) return false;
     const size_t tiles_yz = (size_t)(ny / MTY) * (nz / MTZ);

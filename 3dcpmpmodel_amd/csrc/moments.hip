@@ -106,10 +106,6 @@ __device__ __forceinline__ unsigned mom_site(const DevParams &P, int y, int z) {
 // (((x * tiles + tile) * 2 + s) * 12 + k) * TY + r.  A neighbour in z reads its halo there
 // instead of one value from each of 12 * TY lines.
 
-template <class TC> __device__ __forceinline__ const TC *rates_of(const DevParams &P);
-template <> __device__ __forceinline__ const double *rates_of<double>(const DevParams &P) { return P.ts; }
-template <> __device__ __forceinline__ const float *rates_of<float>(const DevParams &P) { return P.tsf; }
-
 template <class TF, class TS, class TC>
 struct StepArgs {
     const TF *fin;        // populations (IN_P) or
@@ -124,18 +120,6 @@ struct StepArgs {
     TS *uout;             // adjoint tape: u, grad mu, grad rho (DIAG, may be null)
     int ntz, nty, xc;
 };
-
-// address of element i of a plane whose base is uniform over the wave: the offset stays in
-// 32 bits (a plane of at most 2^31 / 19 values of 8 bytes fits), so the access takes the
-// scalar-base form and no 64-bit address is kept per lane
-template <class T>
-__device__ __forceinline__ T *lane_at(T *base, unsigned i) {
-    using C = std::conditional_t<std::is_const<T>::value, const char, char>;
-    // an empty asm makes the offset a value of this use: hoisted out of the x loop it is
-    // kept zero-extended in two registers and spills
-    asm volatile("" : "+v"(i));
-    return (T *)((C *)base + i * (unsigned)sizeof(T));
-}
 
 enum { kPlain, kQp, kGuo };   // force term: exact difference, with Qp, Guo (Qp if on)
 
@@ -315,9 +299,9 @@ __global__ void __launch_bounds__(TL::NT, sizeof(TC) == 4 ? 4 : 2) k_moment_step
             if (FC != kPlain && P.qp_on) {
                 TC qp[Q];
                 qp_terms(gr[0], gr[1], gr[2], (TC)P.K1, (TC)P.K2, qp);
-                collide_moments<TC, true, FC == kGuo>(m, r, Fx, Fy, Fz, rates_of<TC>(P), qp, out, u);
+                collide_moments<TC, true, FC == kGuo>(m, r, Fx, Fy, Fz, rates<TC>(P), qp, out, u);
             } else {
-                collide_moments<TC, true, FC == kGuo>(m, r, Fx, Fy, Fz, rates_of<TC>(P), (const TC *)nullptr, out, u);
+                collide_moments<TC, true, FC == kGuo>(m, r, Fx, Fy, Fz, rates<TC>(P), (const TC *)nullptr, out, u);
             }
             if (post) {
 #pragma unroll
@@ -483,10 +467,11 @@ hipError_t launch_form(cpmp_ctx *c, bool in_p, bool out_p, void *mv, TS *uout) {
 // Planes per workgroup.  A chunk of n planes collides n + 2 and loads 7 planes of rho and
 // mu before its first (together about 4 planes' time), and the launch takes as many
 // rounds as its workgroups need places on the device (2 per CU with 4-byte arithmetic,
-// 1 with 8-byte: LDS; twice as many of the one-row tiles' 4 waves), so the chunk length that minimises rounds * (n + 4) is taken.  Within
-// 3 % of the best of a sweep over 1..24 planes on 13 lattices (64^3 FP64 4: 36.5 us, 8: 54.6;
-// 128^3 FP32 11: 87.5, 4: 104, 24: 134; 256^3 FP32 32: 533, 43: 568).
-// CPMP_XC overrides.
+// 1 with 8-byte: LDS; twice as many of the one-row tiles' 4 waves), so the chunk length that
+// minimises rounds * (n + 4) is taken.  In a sweep over 1..128 planes on 14 lattices in three
+// forms, kept under profiles/, it is the best in 34 of 42 runs and within 9 % of it in all (us
+// per step: 64^3 FP64 4: 32.7, 2: 43.5, 8: 46.6; 128^3 FP32 12: 77, 4: 90, 24: 118; 256^3 FP32
+// 32: 491, 16: 520, 43: 562; 3001x1x501 FP64 18: 101, 8: 112, 32: 142).  CPMP_XC overrides.
 int moment_chunk(int nx, int ny, int nz, int form) {
     if (const char *e = std::getenv("CPMP_XC")) {
         const int v = std::atoi(e);

@@ -17,9 +17,10 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_HBM_GBS = 8000.0     # MI355X HBM3E, AMD published
-# bytes per node that a step within a run reads and writes of the state: 13 numbers (density
-# and 12 moments) each way in the precision they are computed in; FP16 storage: 19 populations
-STATE_BYTES = {"fp64": 2 * 13 * 8, "fp32": 2 * 13 * 4, "fp32a": 2 * 13 * 4, "fp16": 2 * 19 * 2}
+# bytes per node that a step within a run reads and writes of the state: 12 moments in the
+# precision they are computed in and the density in that of its storage, each way; FP16
+# storage: 19 populations
+STATE_BYTES = {"fp64": 2 * 13 * 8, "fp32": 2 * 13 * 4, "fp32a": 2 * (12 * 4 + 8), "fp16": 2 * 19 * 2}
 G_RKE, L_RKE = 0.0319804, 8.25467   # CoCurve_RKE_2.txt Tr=0.60 row times Rc
 
 

@@ -279,7 +279,9 @@ int cpmp_adjoint_plan(cpmp_ctx *ctx, const cpmp_adj_desc *d, cpmp_adj_plan *plan
 int cpmp_kernel_times(cpmp_ctx *ctx, int nsteps, double *ms_per_launch, int *launches_per_step);
 /* Elapsed device time (ms) of nsteps whole steps on the context's stream. */
 int cpmp_time_steps(cpmp_ctx *ctx, int nsteps, double *ms);
-/* Algorithmic bytes per node per step of the current form (2*19*sizeof(population)). */
+/* Bytes per node that a step on populations reads and writes in the current form
+   (2*19*sizeof(population)).  Within a call, lattices that carry moments from step to step
+   move less: 12 moments in the precision of the arithmetic and the density, each way. */
 double cpmp_algorithmic_bytes_per_node(cpmp_ctx *ctx);
 
 const char *cpmp_last_error(void);

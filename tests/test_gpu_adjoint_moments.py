@@ -11,9 +11,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("lo,hi,scheme", [(3, 3, 1), (4, 3, 0)])
-def test_adjoint_of_a_lattice_on_moments_matches_the_oracle(cpmp, lo, hi, scheme):
+def test_adjoint_of_a_lattice_on_moments_matches_the_oracle(cpmp, monkeypatch, lo, hi, scheme):
     """92 160 nodes: J and the gradients against the oracle's reverse mode, all steps taped,
     recomputed from checkpoints, and both with a call before it on the same context"""
+    monkeypatch.delenv("CPMP_COLLIDE", raising=False)
     dims, nsteps = (48, 48, 40), 8
     kw, rho0, mu_lo, mu_hi, target = ta.small_case(cpmp, *dims)
     kw.update(nwall=lo, nwall_hi=hi, wall_scheme=scheme)
