@@ -1234,29 +1234,29 @@ template <class TS> static const TS *ref_buffer(const cpmp_ctx *c) {
 
 // Thin lattices of 80 000 nodes and more that the population kernels step faster than the
 // moments do: the 12 x 32 tile repeats the periodic rows of ny = 2..4 in most of its lanes.
-// us per call of 20 steps, population kernels against moments.
+// us per call of 20 steps, population kernels against moments (more under profiles/).
 static bool thin_lattice(const cpmp_params &p) {
     const bool node = node_collide(p.nx, p.ny, p.nz, p.form);
     const long long n = (long long)p.nx * p.ny * p.nz;
     auto up = [](long long a, long long b) { return (a + b - 1) / b; };
     if (p.form == CPMP_FORM_FP64) {
         // one plane: three collided for one stepped, and the places of FP64 (256 workgroups) hold
-        // one round (1x146x582 493 / 417, 1x300x400 602 / 675, 1x700x700 1428 / 1876)
+        // one round (1x146x582 482 / 418, 1x300x400 596 / 678, 1x700x700 1396 / 1885)
         if (p.nx == 1) return up(p.ny, 12) * up(p.nz, 32) > 256;
-        // against one thread per node, in lanes of its 4 x 64 blocks (428x2x225 878 / 1300, 922x3x36
-        // 672 / 849, 575x3x97 820 / 971, 1930x4x34 1252 / 1470; 981x3x70 1191 / 1164, 2.25 times the
-        // lanes; 300x5x60 597 / 538)
+        // against one thread per node, in lanes of its 4 x 64 blocks: 428x2x225 777 / 1304, 922x3x36
+        // 590 / 851, 575x3x97 760 / 976, 1930x4x34 1122 / 1474, and with 2.25 times the lanes 981x3x70
+        // 1074 / 1170, but with 4 rows 0.92 to 0.98 of the time (826x4x70); 300x5x60 598 / 538
         const long long lanes = up(p.ny, 12) * 12 * up(p.nz, 32) * 32, node_lanes = up(p.ny, 4) * 4 * up(p.nz, 64) * 64;
-        if (node) return p.ny == 2 || (p.ny <= 4 && 2 * lanes >= 5 * node_lanes);
-        // against the population march with long chunks (496x2x1368, 16 planes: 6776 / 6973;
-        // 295x2x1311, 8 planes: 3986 / 3888)
+        if (node) return p.ny == 2 || (p.ny == 3 && lanes >= 2 * node_lanes) || (p.ny == 4 && 2 * lanes >= 5 * node_lanes);
+        // against the population march with long chunks: 496x2x1368, 16 planes, 6365 / 6975; of 8
+        // planes 0.91 to 1.04
         return p.ny == 2 && march_chunk_rule(p.nx, p.ny, p.nz, p.form) >= 16;
     }
     if (p.ny != 2) return false;
-    // 544x2x83 607 / 654, 40x2x1267 598 / 643; 489x2x197 1178 / 890
+    // 544x2x83 563 / 657, 40x2x1267 540 / 645; 489x2x197 1063 / 891
     if (p.form == CPMP_FORM_FP32A) return node && n < 160000;
-    // march chunks of 4 and more: 496x2x1368 2968 / 3518, 212x2x1264 1486 / 1580; of 2: 562x2x996 0.80
-    // of the time; of 1: 100x2x1067 1189 / 816
+    // march chunks of 4 and more: 496x2x1368 2727 / 3501, 2017x2x118 1479 / 1481; of 2: 562x2x996
+    // 3138 / 2825; of 1: 100x2x1067 1012 / 814
     return march_chunk_rule(p.nx, p.ny, p.nz, p.form) >= 4;
 }
 

@@ -136,7 +136,8 @@ def test_the_switches_select_the_path(cpmp, monkeypatch, form):
 
 @pytest.mark.parametrize("form,dims,moments", [
     ("fp64", (428, 2, 225), False), ("fp64", (873, 2, 263), True), ("fp64", (496, 2, 1368), False),
-    ("fp64", (922, 3, 36), False), ("fp64", (981, 3, 70), True), ("fp64", (968, 4, 34), False),
+    ("fp64", (922, 3, 36), False), ("fp64", (981, 3, 70), False), ("fp64", (946, 3, 298), True),
+    ("fp64", (968, 4, 34), False), ("fp64", (826, 4, 70), True),
     ("fp64", (300, 5, 60), True), ("fp64", (1, 300, 400), False), ("fp64", (1, 146, 582), True),
     ("fp32a", (544, 2, 83), False), ("fp32a", (489, 2, 197), True), ("fp32a", (922, 3, 36), True),
     ("fp32", (212, 2, 1264), False), ("fp32", (562, 2, 996), True), ("fp32", (100, 2, 1067), True),
