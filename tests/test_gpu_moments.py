@@ -98,16 +98,21 @@ def test_moment_runs_split_into_calls_are_bitwise_the_same(cpmp, monkeypatch, tm
 @pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[10], CASES[12]], ids=lambda c: "x".join(map(str, c[0])))
 def test_fp32_arithmetic_form_sums_the_density_in_fp64(cpmp, monkeypatch, case):
     """FP64 storage with FP32 arithmetic: the stored density is the FP64 sum of the 19
-    values that the next step pulls, whichever step of a call wrote it.  Two sums of 19
-    terms in any order differ by at most 2 * 18 * 2^-53 of the sum of magnitudes."""
+    values that the next step pulls, from the sums of two (one rounding of 2^-24 each) and
+    of four (two) that the moments use anyway.  Sums of all 19 in FP32 err by 0.3 to 0.5
+    of 2^-24 of the density on average, these by 0.1."""
     a = lattice(cpmp, monkeypatch, case, "fp32a", "moments")
     fluid = a.get("type") == 1
+    u = 2.0 ** -24
     for n in (1, 4):
         a.step(n)
         f = a.get("f").reshape(19, -1)[:, fluid]
-        err = np.max(np.abs(a.get("rho")[fluid] - f.sum(axis=0)) / np.abs(f).sum(axis=0))
-        print(f"[moments] {case[0]} fp32a density: {err:.2e}", flush=True)
-        assert err <= 36 * 2.0 ** -53
+        err = np.abs(a.get("rho")[fluid] - f.sum(axis=0))
+        bound = u * (np.abs(f[1:7]).sum(axis=0) + 2 * np.abs(f[7:]).sum(axis=0)) + 36 * 2.0 ** -53 * np.abs(f).sum(axis=0)
+        mean = float(np.mean(err / f.sum(axis=0))) / u
+        print(f"[moments] {case[0]} fp32a density: {np.max(err / bound):.2f} of the bound, mean {mean:.2f} 2^-24", flush=True)
+        assert np.all(err <= bound)
+        assert mean < 0.2
     a.close()
 
 
