@@ -9,11 +9,15 @@ import oracle_lib as orc
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("collide", ["auto", "moments"])
 @pytest.mark.parametrize("scheme", [0, 1])
 @pytest.mark.parametrize("lo,hi", [(1, 2), (4, 1), (2, 4), (4, 4), (5, 3), (0, 6)])
-def test_wall_fill_and_its_adjoint_at_every_depth(cpmp, lo, hi, scheme):
+def test_wall_fill_and_its_adjoint_at_every_depth(cpmp, monkeypatch, lo, hi, scheme, collide):
     """two steps (solid density and potential included), then the adjoint of five, on a
-    lattice the 16 x 16 column tiles do not cover"""
+    lattice the 16 x 16 column tiles do not cover, with the per-node collide it takes and on
+    moments"""
+    if collide != "auto":
+        monkeypatch.setenv("CPMP_COLLIDE", collide)
     dims = (18, 17, 26)
     kw = dict(eos="VDW", tr=0.8, nwall=lo, nwall_hi=hi, wall_scheme=scheme)
     rng = np.random.default_rng(4)
