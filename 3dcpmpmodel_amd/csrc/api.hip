@@ -11,7 +11,6 @@
 #include <cstdio>
 #include <cstring>
 #include <fstream>
-#include <map>
 #include <mutex>
 #include <sstream>
 #include <string>
@@ -35,31 +34,35 @@ int set_error(int code, const char *fmt, ...) {
 // what the library holds of a device beside its contexts' own buffers
 namespace {
 struct DeviceShare {
-    int contexts = 0;         // open on the device
-    char *idle = nullptr;     // the adjoint workspace no call is using
-    size_t idle_bytes = 0;
+    int contexts;         // open on the device
+    char *idle;           // the adjoint workspace no call is using
+    size_t idle_bytes;
 };
+constexpr int kShares = 64;   // devices from here on keep nothing
 std::mutex g_share_mu;
-std::map<int, DeviceShare> g_share;
+DeviceShare g_share[kShares] = {};
+DeviceShare *share(int device) { return device >= 0 && device < kShares ? &g_share[device] : nullptr; }
 }  // namespace
 
 char *workspace_take(int device, size_t *bytes) {
     std::lock_guard<std::mutex> lock(g_share_mu);
-    DeviceShare &s = g_share[device];
-    char *p = s.idle;
-    *bytes = s.idle_bytes;
-    s.idle = nullptr;
-    s.idle_bytes = 0;
+    DeviceShare *s = share(device);
+    char *p = s ? s->idle : nullptr;
+    *bytes = s ? s->idle_bytes : 0;
+    if (s) {
+        s->idle = nullptr;
+        s->idle_bytes = 0;
+    }
     return p;
 }
 
 void workspace_give(int device, char *block, size_t bytes) {
     {
         std::lock_guard<std::mutex> lock(g_share_mu);
-        DeviceShare &s = g_share[device];
-        if (!s.idle || s.idle_bytes < bytes) {
-            std::swap(s.idle, block);
-            std::swap(s.idle_bytes, bytes);
+        DeviceShare *s = share(device);
+        if (s && (!s->idle || s->idle_bytes < bytes)) {
+            std::swap(s->idle, block);
+            std::swap(s->idle_bytes, bytes);
         }
     }
     if (block) (void)hipFree(block);
@@ -67,7 +70,8 @@ void workspace_give(int device, char *block, size_t bytes) {
 
 size_t workspace_idle(int device) {
     std::lock_guard<std::mutex> lock(g_share_mu);
-    return g_share[device].idle_bytes;
+    const DeviceShare *s = share(device);
+    return s ? s->idle_bytes : 0;
 }
 
 size_t workspace_release(int device) {
@@ -93,16 +97,16 @@ hipError_t device_malloc(int device, void **p, size_t n) {
 static void context_opened(cpmp_ctx *c) {
     std::lock_guard<std::mutex> lock(g_share_mu);
     c->open = true;
-    ++g_share[c->p.device].contexts;
+    if (DeviceShare *s = share(c->p.device)) ++s->contexts;
 }
 
 // the last context of a device takes the kept workspace with it
 static void context_closed(cpmp_ctx *c) {
     if (!c->open) return;
-    bool last;
+    bool last = false;
     {
         std::lock_guard<std::mutex> lock(g_share_mu);
-        last = --g_share[c->p.device].contexts == 0;
+        if (DeviceShare *s = share(c->p.device)) last = --s->contexts == 0;
     }
     if (last) workspace_release(c->p.device);
 }

@@ -130,10 +130,11 @@ __global__ void __launch_bounds__(TPB) k_wall(const DevParams P, TS *__restrict_
 
 // The same fill in one launch for walls of at most R (<= 4) layers (any depth with the
 // simple scheme, which reads the first fluid layer only).  With the layered scheme layer
-// lo-d is A^d applied to the first fluid layer, A the diagonal average above, so a 16 x 16 tile of columns needs the fluid layer on the tile
-// plus a halo of R columns.  The workgroup stages that patch in LDS and recomputes
-// the layers on shrinking patches with the same arithmetic (including the rounding
-// to the storage type) as the pass kernels, so the results are identical.
+// lo-d is A^d applied to the first fluid layer, A the diagonal average above, so a 16 x 16
+// tile of columns needs the fluid layer on the tile plus a halo of R columns.  The workgroup
+// stages that patch in LDS and recomputes the layers on shrinking patches with the same
+// arithmetic (including the rounding to the storage type) as the pass kernels, so the
+// results are identical.
 // blockIdx.z selects the wall (0: bottom, 1: top).
 
 template <int R, class TS>
